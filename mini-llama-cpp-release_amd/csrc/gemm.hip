@@ -12,7 +12,8 @@
 //     workgroup of the split writes one contiguous row, and a GEMM chunk reads
 //     a token's four blocks as 512 contiguous bytes (against block-major
 //     storage: 4096 x 4096 Q4_0 at 512 tokens 68.3 -> 66.8 us per call).
-//  2. gemm: v_mfma_f32_16x16x32_f16 with A = X fragments (16 tokens x 32 k,
+//  2. gemm (more than 128 tokens: the large-tile kernel of gemm_tile.h, the same
+//     products on v_mfma_f32_32x32x16_f16): v_mfma_f32_16x16x32_f16 with A = X fragments (16 tokens x 32 k,
 //     hi then lo) and B = weight fragments (32 k x 16 weight rows) holding the
 //     block's integer codes as exact fp16 values (q, q - 8 or the Q8_0 byte).
 //     One block is one MFMA K step; each block's product starts from zero and is
@@ -35,6 +36,7 @@
 // Weight rows are read as dwords of 2-block pairs (36 / 68 / 40 bytes), which
 // needs an even block count per row; other shapes use the GEMV kernels per row.
 
+#include "gemm_tile.h"
 #include "mlq_kernels.h"
 #include "xsplit_device.h"
 
@@ -46,11 +48,6 @@
 
 namespace mlq {
 namespace {
-
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ float h_lo(uint32_t v) { return (float)__builtin_bit_cast(h2_t, v).x; }
 __device__ __forceinline__ float h_hi(uint32_t v) { return (float)__builtin_bit_cast(h2_t, v).y; }
@@ -76,7 +73,7 @@ __device__ __forceinline__ int slot_k(int g, int j) {
 // max|x| of the row, then the scaled split), so rows up to 16 384 elements are
 // read once; longer rows re-read the rest (L2 hits).  The split itself is
 // xsplit_device.h's, which kernels producing a GEMM input also use.
-template <int QT>
+template <int QT, bool PACK>
 __global__ __launch_bounds__(256) void xsplit_kernel(const float* __restrict__ x, int N, int K,
                                                      int nb, int npad, _Float16* __restrict__ xs,
                                                      float* __restrict__ bsum,
@@ -112,7 +109,7 @@ __global__ __launch_bounds__(256) void xsplit_kernel(const float* __restrict__ x
 #pragma unroll
     for (int c = 0; c < kXsCache; ++c) load16(threadIdx.x + 256 * c, cache[c]);
     if (nhb <= 256 * kXsCache) {
-        xsplit_emit_row<QT, kXsCache>(n, nb, cache, xs, bsum, scale, red);
+        xsplit_emit_row<QT, kXsCache, PACK>(n, nb, cache, xs, bsum, scale, red);
         return;
     }
     float mx = 0.0f;
@@ -132,12 +129,12 @@ __global__ __launch_bounds__(256) void xsplit_kernel(const float* __restrict__ x
     if (threadIdx.x == 0) scale[n] = sc;
     const int iters = (nhb + 255) / 256;  // uniform across the workgroup
 #pragma unroll
-    for (int c = 0; c < kXsCache; ++c) xsplit_emit_half<QT>(n, nb, threadIdx.x + 256 * c, cache[c], inv, xs, bsum);
+    for (int c = 0; c < kXsCache; ++c) xsplit_emit_half<QT, PACK>(n, nb, threadIdx.x + 256 * c, cache[c], inv, xs, bsum);
     for (int it = kXsCache; it < iters; ++it) {
         float v[16];
         const int hb = threadIdx.x + 256 * it;
         load16(hb, v);
-        xsplit_emit_half<QT>(n, nb, hb, v, inv, xs, bsum);
+        xsplit_emit_half<QT, PACK>(n, nb, hb, v, inv, xs, bsum);
     }
 }
 
@@ -150,11 +147,6 @@ struct WFrag {
     float m;
 };
 
-__device__ __forceinline__ uint32_t bias_sub(uint32_t v, uint32_t neg_bias2) {
-    const h2_t r = __builtin_bit_cast(h2_t, v) + __builtin_bit_cast(h2_t, neg_bias2);
-    return __builtin_bit_cast(uint32_t, r);
-}
-
 // Q4 nibble dword (bytes 4g..4g+3 of qs) -> 8 fp16 codes in slot order.
 __device__ __forceinline__ f16x8 nibbles_to_f16(uint32_t q, uint32_t neg_bias2, uint32_t mask,
                                                 uint32_t magic) {
@@ -164,18 +156,6 @@ __device__ __forceinline__ f16x8 nibbles_to_f16(uint32_t q, uint32_t neg_bias2, 
     const uint32_t t3 = ((q >> 12) & mask) | magic;
     const u32x4 r{bias_sub(t0, neg_bias2), bias_sub(t1, neg_bias2), bias_sub(t2, neg_bias2),
                   bias_sub(t3, neg_bias2)};
-    return __builtin_bit_cast(f16x8, r);
-}
-
-// Q8_0 byte dwords (qs bytes 8g..8g+7) -> 8 fp16 codes.
-__device__ __forceinline__ f16x8 bytes_to_f16(uint32_t a, uint32_t b, uint32_t neg_bias2) {
-    const uint32_t ax = a ^ 0x80808080u;
-    const uint32_t bx = b ^ 0x80808080u;
-    const uint32_t mb = 0x64646464u;
-    const u32x4 r{bias_sub(__builtin_amdgcn_perm(mb, ax, 0x04010400u), neg_bias2),
-                  bias_sub(__builtin_amdgcn_perm(mb, ax, 0x04030402u), neg_bias2),
-                  bias_sub(__builtin_amdgcn_perm(mb, bx, 0x04010400u), neg_bias2),
-                  bias_sub(__builtin_amdgcn_perm(mb, bx, 0x04030402u), neg_bias2)};
     return __builtin_bit_cast(f16x8, r);
 }
 
@@ -505,22 +485,19 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_stream_kernel(
 //    with coalesced 8-byte loads, P chunks ahead, into registers, and parks it
 //    in a wave-private LDS buffer; MFMA B fragments are read back from there.
 //  * x, one chunk ahead, into a shared LDS buffer of A fragments (slot order
-//    of the weight codes), from one of two sources:
-//    XS: the x split by xsplit_kernel (per-token power-of-two scale, fp16 hi +
-//        lo in fragment order, Q4_1 block sums): a plain copy;
-//    !XS: the f32 x itself (small batches, where a second launch would cost
-//        more than the split): the workgroup picks a power-of-two scale per
-//        (token, chunk) that puts the chunk's max|x| in [2^13, 2^14) and
-//        splits every scaled element into fp16 hi + lo.
+//    of the weight codes): the f32 x itself (small batches, where a second
+//    launch would cost more than the split); the workgroup picks a
+//    power-of-two scale per (token, chunk) that puts the chunk's max|x| in
+//    [2^13, 2^14) and splits every scaled element into fp16 hi + lo.
 //  * MFMAs: per block, hi then lo into a zeroed tile, then the block scale
-//    d (+ m * sum(x') for Q4_1) times the tile into the accumulator (!XS: into
-//    a chunk accumulator that is scaled back by the chunk's inverse scale).
+//    d (+ m * sum(x') for Q4_1) times the tile into a chunk accumulator that is
+//    scaled back by the chunk's inverse scale.
 // K is split across workgroups only when the tiles alone would not fill the
 // CUs; the splits of a tile are adjacent in launch order.  Each split stores
 // its partial tile with write-through stores and counts in; the workgroup
-// that completes the count adds the partials in split order (deterministic),
-// applies the token scale and writes y.  Needs nb % 4 == 0 (8-byte aligned
-// chunk rows), K == 32 nb and (!XS) a 16-byte aligned x.
+// that completes the count adds the partials in split order (deterministic)
+// and writes y.  Needs nb % 4 == 0 (8-byte aligned
+// chunk rows), K == 32 nb and a 16-byte aligned x.
 constexpr int kChunkBlocks = 4;
 
 template <int QT> struct ChunkFmt;
@@ -528,14 +505,14 @@ template <> struct ChunkFmt<1> { static constexpr int BB = 34, U = 17, WROW = 13
 template <> struct ChunkFmt<2> { static constexpr int BB = 18, U = 9, WROW = 72; };
 template <> struct ChunkFmt<3> { static constexpr int BB = 20, U = 10, WROW = 80; };
 
-template <int QT, int RW, int TT, bool XS>
+template <int QT, int RW, int TT>
 struct ChunkLds {
     static constexpr int BN = 16 * TT;
     static constexpr int w_wave = RW * 16 * ChunkFmt<QT>::WROW;  // one buffer of one wave
     static constexpr int w_bytes = 2 * 4 * w_wave;                 // [buffer][wave][row][WROW]
     static constexpr int x_halves = kChunkBlocks * BN * kXRowHalves;  // [block][token][72]
-    // + (!XS) inverse scales [BN] + (Q4_1) block sums [block][BN]
-    static constexpr int sums_off = x_halves * 2 + (XS ? 0 : BN * 4);
+    // + inverse scales [BN] + (Q4_1) block sums [block][BN]
+    static constexpr int sums_off = x_halves * 2 + BN * 4;
     static constexpr int x_buf = sums_off + (QT == 3 ? kChunkBlocks * BN * 4 : 0);
     static constexpr int bytes = w_bytes + 2 * x_buf;
 };
@@ -548,10 +525,7 @@ constexpr int kCoherent = 16;  // sc1: write through / read from the point of co
 
 struct ChunkArgs {
     const uint8_t* W;
-    const float* x;         // !XS: f32 x [N][K]
-    const _Float16* xs;     // XS: split x [npad][nb][64] (token-major)
-    const float* bsum;      // XS, Q4_1: [npad][nb]
-    const float* xscale;    // XS: [npad]
+    const float* x;         // f32 x [N][K]
     float* y;
     float* part;
     uint32_t part_bytes;
@@ -574,15 +548,14 @@ struct ChunkArgs {
     int xcd_br, xcd_row_outer;
 };
 
-template <int QT, int RW, int TT, int P, bool XS>
+template <int QT, int RW, int TT, int P>
 __global__ __launch_bounds__(kGemmThreads) void gemm_chunk_kernel(const ChunkArgs a) {
-    using L = ChunkLds<QT, RW, TT, XS>;
+    using L = ChunkLds<QT, RW, TT>;
     using F = ChunkFmt<QT>;
     constexpr int BN = L::BN;
-    constexpr int TPT = kGemmThreads / BN;  // !XS: x-split threads per token
-    constexpr int EPT = 128 / TPT;          // !XS: elements per thread per chunk (8, 16 or 32)
-    constexpr int XU = kChunkBlocks * BN * 8 / kGemmThreads;  // XS: 16-byte x units per thread per chunk
-    constexpr int XR = XS ? XU : EPT / 4;   // x registers (float4 / 16-byte units) per thread
+    constexpr int TPT = kGemmThreads / BN;  // x-split threads per token
+    constexpr int EPT = 128 / TPT;          // elements per thread per chunk (8 or 16)
+    constexpr int XR = EPT / 4;             // x registers (float4) per thread
     constexpr int WU = RW * 16 * F::U;      // weight units per wave per chunk
     constexpr int NWL = (WU + 63) / 64;     // weight loads per lane per chunk
     extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -639,33 +612,15 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_chunk_kernel(const ChunkArg
     const bool last_ok = lane + 64 * (NWL - 1) < WU;  // the last load is partial when 64 does not divide WU
     constexpr size_t kChunkBytes = static_cast<size_t>(kChunkBlocks) * F::BB;
 
-    // !XS: x slice of this thread: token tok, elements e0 .. e0 + EPT - 1 of the chunk.
+    // x slice of this thread: token tok, elements e0 .. e0 + EPT - 1 of the chunk.
     const int tok = tid / TPT;
     const int e0 = (tid % TPT) * EPT;
     const bool tok_ok = n_base + tok < N;
-    const float* xrow = XS ? nullptr
-                           : a.x + static_cast<size_t>(tok_ok ? n_base + tok : 0) * a.K +
-                                 static_cast<size_t>(c0) * 128 + e0;
-    // XS: unit v = tid + 256 i -> (token, block j, 16-byte column q) of the
-    // chunk: a token's four blocks are 512 contiguous bytes of the split x.
-    uint32_t xoff[XS ? XU : 1];
-    int xl_off[XS ? XU : 1];
-    if (XS) {
-#pragma unroll
-        for (int i = 0; i < XU; ++i) {
-            const int v = tid + kGemmThreads * i;
-            const int q = v % 8;
-            const int j = (v / 8) % kChunkBlocks;
-            const int tk = v / (8 * kChunkBlocks);
-            xoff[i] = (static_cast<uint32_t>(n_base + tk) * a.nb + j) * 64 + 8 * q;  // halves, from the chunk's block 0
-            xl_off[i] = ((j * BN + tk) * kXRowHalves + 8 * q) * 2;                      // bytes
-        }
-    }
-    const bool sum_lane = XS && QT == 3 && tid < kChunkBlocks * BN;
+    const float* xrow =
+        a.x + static_cast<size_t>(tok_ok ? n_base + tok : 0) * a.K + static_cast<size_t>(c0) * 128 + e0;
 
     uint2 wreg[P][NWL];
     u32x4 xreg[XR];
-    float sreg = 0.0f;
     auto load_w = [&](int c, uint2 (&wr)[NWL]) {
         const uint8_t* wc = wsplit + static_cast<size_t>(c) * kChunkBytes;
 #pragma unroll
@@ -679,29 +634,12 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_chunk_kernel(const ChunkArg
         }
     };
     auto load_x = [&](int c) {
-        if (XS) {
-            const int b = (c0 + c) * kChunkBlocks;
-            const _Float16* src = a.xs + static_cast<size_t>(b) * 64;
+        const u32x4* src = reinterpret_cast<const u32x4*>(xrow + static_cast<size_t>(c) * 128);
 #pragma unroll
-            for (int i = 0; i < XU; ++i) xreg[i] = *reinterpret_cast<const u32x4*>(src + xoff[i]);
-            if (QT == 3) {
-                const int t = sum_lane ? tid : 0;
-                sreg = a.bsum[static_cast<size_t>(n_base + t % BN) * a.nb + b + t / BN];
-            }
-        } else {
-            const u32x4* src = reinterpret_cast<const u32x4*>(xrow + static_cast<size_t>(c) * 128);
-#pragma unroll
-            for (int i = 0; i < XR; ++i) xreg[i] = src[i];
-        }
+        for (int i = 0; i < XR; ++i) xreg[i] = src[i];
     };
     auto put_x = [&](int buf) {
         char* xb = smem + L::w_bytes + buf * L::x_buf;
-        if (XS) {
-#pragma unroll
-            for (int i = 0; i < XU; ++i) *reinterpret_cast<u32x4*>(xb + xl_off[i]) = xreg[i];
-            if (sum_lane) reinterpret_cast<float*>(xb + L::sums_off)[tid] = sreg;
-            return;
-        }
         _Float16* xl = reinterpret_cast<_Float16*>(xb);
         float* sl = reinterpret_cast<float*>(xb + L::x_halves * 2);
         float v[EPT];
@@ -775,7 +713,7 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_chunk_kernel(const ChunkArg
         const char* xb = smem + L::w_bytes + buf * L::x_buf;
         const _Float16* xl = reinterpret_cast<const _Float16*>(xb);
         const float* ssum = reinterpret_cast<const float*>(xb + L::sums_off);
-        f32x4 cacc[XS ? 1 : RW][XS ? 1 : TT];
+        f32x4 cacc[RW][TT];
         f32x4 bprev[RW][TT];
         float dprev[RW], mprev[RW];
         f32x4 svprev[TT];
@@ -786,16 +724,10 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_chunk_kernel(const ChunkArg
                 for (int t = 0; t < TT; ++t)
 #pragma unroll
                     for (int q = 0; q < 4; ++q) {
-                        if (XS) {
-                            float v = __builtin_fmaf(dprev[r], bprev[r][t][q], acc[r][t][q]);
-                            if (QT == 3) v = __builtin_fmaf(mprev[r], svprev[t][q], v);
-                            acc[r][t][q] = v;
-                        } else {
-                            float v = jb == 0 ? dprev[r] * bprev[r][t][q]
-                                              : __builtin_fmaf(dprev[r], bprev[r][t][q], cacc[r][t][q]);
-                            if (QT == 3) v = __builtin_fmaf(mprev[r], svprev[t][q], v);
-                            cacc[r][t][q] = v;
-                        }
+                        float v = jb == 0 ? dprev[r] * bprev[r][t][q]
+                                          : __builtin_fmaf(dprev[r], bprev[r][t][q], cacc[r][t][q]);
+                        if (QT == 3) v = __builtin_fmaf(mprev[r], svprev[t][q], v);
+                        cacc[r][t][q] = v;
                     }
         };
 #pragma unroll
@@ -844,17 +776,14 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_chunk_kernel(const ChunkArg
             }
         }
         epilogue(kChunkBlocks - 1);
-        if (!XS) {
-            const float* sl = reinterpret_cast<const float*>(xb + L::x_halves * 2);
+        const float* sl = reinterpret_cast<const float*>(xb + L::x_halves * 2);
 #pragma unroll
-            for (int t = 0; t < TT; ++t) {
-                const f32x4 s4 = *reinterpret_cast<const f32x4*>(sl + t * 16 + 4 * g);
+        for (int t = 0; t < TT; ++t) {
+            const f32x4 s4 = *reinterpret_cast<const f32x4*>(sl + t * 16 + 4 * g);
 #pragma unroll
-                for (int r = 0; r < RW; ++r)
+            for (int r = 0; r < RW; ++r)
 #pragma unroll
-                    for (int q = 0; q < 4; ++q)
-                        acc[r][t][q] = __builtin_fmaf(s4[q], cacc[XS ? 0 : r][XS ? 0 : t][q], acc[r][t][q]);
-            }
+                for (int q = 0; q < 4; ++q) acc[r][t][q] = __builtin_fmaf(s4[q], cacc[r][t][q], acc[r][t][q]);
         }
     };
 
@@ -914,12 +843,6 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_chunk_kernel(const ChunkArg
         }
     }
 
-    // Token scale of output element q of token tile t (XS: the x split's
-    // per-token scale; !XS: already applied per chunk).
-    auto tok_scale = [&](int t, int q) {
-        if (!XS) return 1.0f;
-        return a.xscale[n_base + t * 16 + 4 * g + q];
-    };
     if (a.splits == 1) {
 #pragma unroll
         for (int t = 0; t < TT; ++t)
@@ -927,11 +850,10 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_chunk_kernel(const ChunkArg
             for (int q = 0; q < 4; ++q) {
                 const int n = n_base + t * 16 + 4 * g + q;
                 if (n >= N) continue;
-                const float sn = tok_scale(t, q);
 #pragma unroll
                 for (int r = 0; r < RW; ++r) {
                     const int m = m_base + (wave * RW + r) * 16 + i16;
-                    if (m < M) yg[static_cast<size_t>(n) * M + m] = acc[r][t][q] * sn;
+                    if (m < M) yg[static_cast<size_t>(n) * M + m] = acc[r][t][q];
                 }
             }
         return;
@@ -991,7 +913,7 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_chunk_kernel(const ChunkArg
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             const int n = n_base + t * 16 + 4 * g + q;
-            if (n < N && m < M) yg[static_cast<size_t>(n) * M + m] = sum[k][q] * tok_scale(t, q);
+            if (n < N && m < M) yg[static_cast<size_t>(n) * M + m] = sum[k][q];
         }
     }
     if (tid == 0) __hip_atomic_store(a.tile_count + tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1057,7 +979,7 @@ hipError_t launch_t(const LinearShape& s, const GemmCfg& c, const WsLayout& l, c
     float* scale = reinterpret_cast<float*>(ws + l.scale);
     float* part = c.splits > 1 ? reinterpret_cast<float*>(ws + l.part) : nullptr;
     unsigned* count = reinterpret_cast<unsigned*>(ws + l.count);
-    hipLaunchKernelGGL((xsplit_kernel<QT>), dim3(c.npad), dim3(256), 0, stream, x, s.rows, s.K, s.nb,
+    hipLaunchKernelGGL((xsplit_kernel<QT, false>), dim3(c.npad), dim3(256), 0, stream, x, s.rows, s.K, s.nb,
                        c.npad, xs, bsum, scale);
     dim3 grid((s.M + 64 * RT - 1) / (64 * RT), c.npad / (16 * TT), c.splits);
     constexpr int lds = StreamLds<TT>::bytes;
@@ -1079,22 +1001,17 @@ hipError_t launch_q(const LinearShape& s, const GemmCfg& c, const WsLayout& l, c
 }
 
 // Chunked-kernel configuration (rules from an MI355X sweep of rows per wave,
-// token tile, x split, prefetch depth and K splits at 4096x4096 and
-// 11008x4096, Q4_0 and Q8_0, N = 16 / 64 / 512):
+// token tile, prefetch depth and K splits at 4096x4096 and 11008x4096, Q4_0 and
+// Q8_0, N = 16 / 64):
 //  * up to 16 tokens: 64 rows (one row tile per wave) x 16 tokens per
 //    workgroup, K split until the grid is about 640 workgroups with at least
 //    4 chunks per split (fewer, longer splits beat a larger grid: the split
 //    reduction is a serial tail; short rows keep 2 chunks per split);
-//  * up to 128 tokens: 128 rows x 32 tokens, x split in the kernel;
-//  * more tokens: x split once by xsplit_kernel (the in-kernel split would be
-//    repeated by every row tile), 128 rows x 32 tokens, or x 64 tokens for
-//    Q8_0 from 512 tokens (its 34-byte blocks gain most from fewer weight
-//    passes there; at 256 tokens, and for Q4 throughout, the larger tile's
-//    single workgroup per CU measured slower: 11008 x 4096 Q8_0 N = 256
-//    124.2 against 110.4 us);
-//  * from 32 tokens on, 8 chunks per split unless the tiles alone give every
-//    CU a workgroup (then no K split; with x split once, two splits until
-//    there are two workgroups per CU).
+//  * up to 128 tokens: 128 rows x 32 tokens; from 32 tokens on, 8 chunks per
+//    split unless the tiles alone give every CU a workgroup (then no K split).
+// More tokens run the large-tile kernel (choose_tile); for them this
+// configuration only sizes the workspace (gemm_workspace_bytes), so that the
+// shapes that fit a fixed scratch do not depend on the tile kernel's splits.
 struct ChunkCfg {
     int rw, tt, row_tiles, tok_tiles, splits, cps, npad;
     bool xs;
@@ -1121,7 +1038,6 @@ ChunkCfg choose_chunk(const LinearShape& s) {
     } else if (!c.xs) {
         splits = tiles >= 256 ? 1 : nchunks / 8;
     } else {
-        // N = 256: two splits for 256 tiles (4096 x 4096 Q4_0: 45.2 -> 40.1 us)
         const bool fill = c.tt == 4 ? tiles >= 256 : tiles >= 512;
         splits = fill ? 1 : tiles >= 256 ? 2 : nchunks / 8;
     }
@@ -1137,26 +1053,79 @@ struct ChunkWs {
     size_t xs, bsum, scale, part, part_bytes, total;
 };
 
-ChunkWs chunk_layout(const LinearShape& s, const ChunkCfg& c) {
+ChunkWs ws_layout(const LinearShape& s, bool xs, int npad, size_t part_bytes) {
     auto up = [](size_t v) { return (v + 255) & ~static_cast<size_t>(255); };
     ChunkWs l;
     l.xs = up(static_cast<size_t>(kGemmMaxTiles) * sizeof(unsigned));
-    l.bsum = l.xs + (c.xs ? up(static_cast<size_t>(s.nb) * c.npad * 64 * sizeof(_Float16)) : 0);
-    l.scale = l.bsum + (c.xs ? up(static_cast<size_t>(s.nb) * c.npad * sizeof(float)) : 0);
-    l.part = l.scale + (c.xs ? up(static_cast<size_t>(c.npad) * sizeof(float)) : 0);
-    l.part_bytes = c.splits == 1 ? 0
-                                 : static_cast<size_t>(c.row_tiles) * c.tok_tiles * c.splits *
-                                       (c.rw * c.tt * kGemmThreads * 16);
+    l.bsum = l.xs + (xs ? up(static_cast<size_t>(s.nb) * npad * 64 * sizeof(_Float16)) : 0);
+    l.scale = l.bsum + (xs ? up(static_cast<size_t>(s.nb) * npad * sizeof(float)) : 0);
+    l.part = l.scale + (xs ? up(static_cast<size_t>(npad) * sizeof(float)) : 0);
+    l.part_bytes = part_bytes;
     l.total = l.part + l.part_bytes;
     return l;
 }
 
-size_t chunk_workspace_bytes(const LinearShape& s) { return chunk_layout(s, choose_chunk(s)).total; }
+ChunkWs chunk_layout(const LinearShape& s, const ChunkCfg& c) {
+    return ws_layout(s, c.xs, c.npad,
+                     c.splits == 1 ? 0
+                                   : static_cast<size_t>(c.row_tiles) * c.tok_tiles * c.splits *
+                                         (c.rw * c.tt * kGemmThreads * 16));
+}
 
-// Two weight chunks in flight per wave at every tile shape: at 16 tokens, four
-// (the earlier default) cost 2.5-15 % (4096 x 4096 Q4_0 12.1 -> 11.8 us,
-// 11008 x 4096 Q8_0 26.6 -> 22.5 us): the ring's VGPRs halve the waves per SIMD,
-// and the loop is not waiting on the weights.
+size_t workspace_bytes(const LinearShape& s) {
+    size_t b = layout(s, choose(s)).total;
+    if (chunk_supported(s)) b = std::max(b, chunk_layout(s, choose_chunk(s)).total);
+    return b;
+}
+
+// Large-tile kernel: 128 rows x 64 tokens, eight waves as 2 row halves x 4
+// blocks of a step, three stages.
+template <int QT> using TileShape = Tile<QT, 2, 2, 2, 1, 4, 3>;
+constexpr int kTileM = TileShape<2>::BM, kTileN = TileShape<2>::BN;
+
+struct TileCfg {
+    int row_tiles, tok_tiles, splits, cps, npad;
+    ChunkWs ws;
+};
+
+// K splits of the tile kernel.  One workgroup fills a CU, so the grid runs in
+// ceil(grid / 256) rounds, each about 7 us (launch or start, first copies,
+// reduction over the waves, stores) plus 1.1 us a step of 128 k; a split adds
+// about 5 us (partial tiles to memory and back).  Measured (4096 x 4096 Q4_0, us):
+// 256 tokens 35.2 / 28.1 / 39.1 with 1 / 2 / 4 splits, 512 tokens 41.5 / 59 with 1 / 2.
+TileCfg choose_tile(const LinearShape& s) {
+    TileCfg c;
+    c.row_tiles = (s.M + kTileM - 1) / kTileM;
+    c.tok_tiles = (s.rows + kTileN - 1) / kTileN;
+    c.npad = c.tok_tiles * kTileN;
+    const long long tiles = static_cast<long long>(c.row_tiles) * c.tok_tiles;
+    const int steps = s.nb / kTileBlocks;
+    const size_t most = workspace_bytes(s);
+    c.splits = 0;
+    double best = 0.0;
+    for (int want = 1; want <= 16 && want <= steps; ++want) {
+        const int cps = (steps + want - 1) / want;
+        const int splits = (steps + cps - 1) / cps;
+        if (splits != want || (splits > 1 && (cps < 4 || tiles > kGemmMaxTiles))) continue;
+        const size_t part = splits == 1 ? 0 : static_cast<size_t>(tiles) * splits * (kTileM * kTileN * 4);
+        const ChunkWs ws = ws_layout(s, true, c.npad, part);
+        if (splits > 1 && (ws.total > most || part >= (static_cast<size_t>(1) << 31))) continue;
+        const double rounds = static_cast<double>((tiles * splits + 255) / 256);
+        const double us = rounds * (7.0 + 1.1 * cps) + (splits > 1 ? 5.0 : 0.0);
+        if (c.splits == 0 || us < best) {
+            best = us;
+            c.splits = splits;
+            c.cps = cps;
+            c.ws = ws;
+        }
+    }
+    return c;
+}
+
+bool use_tile(const LinearShape& s) {
+    return chunk_supported(s) && s.rows > 128 && static_cast<size_t>(s.nb) * kTileN * 128 < (static_cast<size_t>(1) << 31);
+}
+
 // Weights of a grouped call: n <= 3 linears with the same qtype, K and rows.
 struct ChunkGroup {
     int n;
@@ -1165,11 +1134,35 @@ struct ChunkGroup {
     int M[3];
 };
 
-template <int QT, int RW, int TT, bool XS, int P = 2>
-hipError_t launch_chunk_t(const LinearShape& s, const ChunkCfg& c, const void* w, const float* x, float* y,
-                          char* ws, hipStream_t stream, const ChunkGroup* grp = nullptr, bool presplit = false) {
-    constexpr int lds = ChunkLds<QT, RW, TT, XS>::bytes;
-    auto kern = gemm_chunk_kernel<QT, RW, TT, P, XS>;
+// Tiles blocked by XCD (one K split; workgroup i runs on XCD i % 8): rows of
+// blocks over the XCDs, and whether the tokens vary fastest inside a block, which
+// keeps the smaller operand of the block (its weights, rows x K, or its split x,
+// 4 bytes per element) resident.  4096 x 4096 Q4_0 at 512 tokens: fabric reads
+// 76.8 -> 52.7 MB per call.
+void xcd_blocks(const LinearShape& s, int row_tiles, int tok_tiles, int bm, int bn, int* br_out, int* row_outer) {
+    *br_out = 0;
+    *row_outer = 0;
+    if ((row_tiles * tok_tiles) % 8 != 0) return;
+    for (int br : {4, 2, 8, 1}) {
+        const int bt = 8 / br;
+        if (row_tiles % br != 0 || tok_tiles % bt != 0) continue;
+        const double wb = static_cast<double>(row_tiles / br) * bm * s.nb * block_bytes(s.qtype);
+        const double xb = static_cast<double>(tok_tiles / bt) * bn * s.K * 4.0;
+        *br_out = br;
+        *row_outer = wb > xb ? 1 : 0;
+        return;
+    }
+}
+
+// Two weight chunks in flight per wave at every tile shape: at 16 tokens, four
+// (the earlier default) cost 2.5-15 % (4096 x 4096 Q4_0 12.1 -> 11.8 us,
+// 11008 x 4096 Q8_0 26.6 -> 22.5 us): the ring's VGPRs halve the waves per SIMD,
+// and the loop is not waiting on the weights.
+template <int QT, int RW, int TT, int P = 2>
+hipError_t launch_chunk_t(const LinearShape& s, const ChunkCfg& c, const float* x, char* ws, hipStream_t stream,
+                          const ChunkGroup& grp) {
+    constexpr int lds = ChunkLds<QT, RW, TT>::bytes;
+    auto kern = gemm_chunk_kernel<QT, RW, TT, P>;
     static bool attr = [&] {
         return hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                                    lds) == hipSuccess;
@@ -1177,77 +1170,86 @@ hipError_t launch_chunk_t(const LinearShape& s, const ChunkCfg& c, const void* w
     if (!attr) return hipErrorInvalidConfiguration;
     const ChunkWs l = chunk_layout(s, c);
     ChunkArgs a;
-    a.W = static_cast<const uint8_t*>(w);
     a.x = x;
-    a.xs = XS ? reinterpret_cast<const _Float16*>(ws + l.xs) : nullptr;
-    a.bsum = XS ? reinterpret_cast<const float*>(ws + l.bsum) : nullptr;
-    a.xscale = XS ? reinterpret_cast<const float*>(ws + l.scale) : nullptr;
-    a.y = y;
     a.part = reinterpret_cast<float*>(ws + l.part);
     a.part_bytes = static_cast<uint32_t>(l.part_bytes);
     a.tile_count = reinterpret_cast<unsigned*>(ws);
-    a.M = s.M, a.N = s.rows, a.K = s.K, a.nb = s.nb, a.npad = c.npad;
+    a.N = s.rows, a.K = s.K, a.nb = s.nb, a.npad = c.npad;
     a.row_tiles = c.row_tiles, a.splits = c.splits, a.chunks_per_split = c.cps;
-    a.W1 = a.W2 = nullptr;
-    a.y1 = a.y2 = nullptr;
-    a.M1 = a.M2 = 0;
-    a.tile1 = a.tile2 = c.row_tiles;
-    a.xcd_br = 0;
-    a.xcd_row_outer = 0;
-    // One K split: block the tiles by XCD (4096 x 4096 Q4_0 at 512 tokens: fabric reads
-    // 76.8 -> 52.7 MB per call, the time unchanged within 1 %).
-    if (c.splits == 1 && (c.row_tiles * c.tok_tiles) % 8 == 0) {
-        for (int br : {4, 2, 8, 1}) {
-            const int bt = 8 / br;
-            if (c.row_tiles % br == 0 && c.tok_tiles % bt == 0) {
-                a.xcd_br = br;
-                // Keep the smaller operand of the block resident: its weights (rows x K)
-                // or its x (tokens x K, split: 4 bytes per element).
-                const double wb = static_cast<double>(c.row_tiles / br) * 64 * RW * s.nb * block_bytes(s.qtype);
-                const double xb = static_cast<double>(c.tok_tiles / bt) * 16 * TT * s.K * 4.0;
-                a.xcd_row_outer = wb > xb ? 1 : 0;
-                break;
-            }
-        }
-    }
-    if (grp != nullptr) {
-        const int bm = 64 * RW;
-        a.W = static_cast<const uint8_t*>(grp->w[0]);
-        a.y = grp->y[0];
-        a.M = grp->M[0];
-        if (grp->n >= 2) {
-            a.W1 = static_cast<const uint8_t*>(grp->w[1]), a.y1 = grp->y[1], a.M1 = grp->M[1];
-            a.tile1 = grp->M[0] / bm;
-        }
-        if (grp->n >= 3) {
-            a.W2 = static_cast<const uint8_t*>(grp->w[2]), a.y2 = grp->y[2], a.M2 = grp->M[2];
-            a.tile2 = a.tile1 + grp->M[1] / bm;
-        }
-    }
-    if (XS && !presplit) {
-        hipLaunchKernelGGL((xsplit_kernel<QT>), dim3(c.npad), dim3(256), 0, stream, x, s.rows, s.K, s.nb, c.npad,
-                           reinterpret_cast<_Float16*>(ws + l.xs), reinterpret_cast<float*>(ws + l.bsum),
-                           reinterpret_cast<float*>(ws + l.scale));
-    }
+    a.xcd_br = a.xcd_row_outer = 0;
+    if (c.splits == 1) xcd_blocks(s, c.row_tiles, c.tok_tiles, 64 * RW, 16 * TT, &a.xcd_br, &a.xcd_row_outer);
+    const int bm = 64 * RW;
+    a.W = static_cast<const uint8_t*>(grp.w[0]), a.y = grp.y[0], a.M = grp.M[0];
+    a.W1 = static_cast<const uint8_t*>(grp.w[1]), a.y1 = grp.y[1], a.M1 = grp.M[1];
+    a.W2 = static_cast<const uint8_t*>(grp.w[2]), a.y2 = grp.y[2], a.M2 = grp.M[2];
+    a.tile1 = grp.n >= 2 ? grp.M[0] / bm : c.row_tiles;
+    a.tile2 = grp.n >= 3 ? a.tile1 + grp.M[1] / bm : c.row_tiles;
     const int grid = c.row_tiles * c.tok_tiles * c.splits;
     hipLaunchKernelGGL(kern, dim3(grid), dim3(kGemmThreads), lds, stream, a);
     return hipGetLastError();
 }
 
 template <int QT>
-hipError_t launch_chunk_q(const LinearShape& s, const ChunkCfg& c, const void* w, const float* x, float* y,
-                          char* ws, hipStream_t stream, const ChunkGroup* grp = nullptr, bool presplit = false) {
-    if (c.tt == 1) return launch_chunk_t<QT, 1, 1, false>(s, c, w, x, y, ws, stream, grp);
-    if (c.tt == 2 && !c.xs) return launch_chunk_t<QT, 2, 2, false>(s, c, w, x, y, ws, stream, grp);
-    if (c.tt == 2) return launch_chunk_t<QT, 2, 2, true>(s, c, w, x, y, ws, stream, grp, presplit);
-    return launch_chunk_t<QT, 2, 4, true>(s, c, w, x, y, ws, stream, grp, presplit);
+hipError_t launch_tile(const LinearShape& s, const float* x, char* ws, hipStream_t stream, const ChunkGroup& grp,
+                       bool presplit) {
+    using T = TileShape<QT>;
+    static_assert(T::BM == kTileM && T::BN == kTileN && T::lds <= 160 * 1024 - 16, "tile");
+    auto kern = gemm_tile_kernel<QT, 2, 2, 2, 1, 4, 3>;
+    static bool attr = [&] {
+        return hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   T::lds) == hipSuccess;
+    }();
+    if (!attr) return hipErrorInvalidConfiguration;
+    const TileCfg c = choose_tile(s);
+    TileArgs a;
+    for (int g = 0; g < 3; ++g) {
+        a.W[g] = static_cast<const uint8_t*>(grp.w[g]);
+        a.y[g] = grp.y[g];
+        a.M[g] = grp.M[g];
+    }
+    a.tile1 = grp.n >= 2 ? grp.M[0] / kTileM : c.row_tiles;
+    a.tile2 = grp.n >= 3 ? a.tile1 + grp.M[1] / kTileM : c.row_tiles;
+    a.xs = reinterpret_cast<const _Float16*>(ws + c.ws.xs);
+    a.bsum = reinterpret_cast<const uint32_t*>(ws + c.ws.bsum);
+    a.xscale = reinterpret_cast<const float*>(ws + c.ws.scale);
+    a.part = reinterpret_cast<float*>(ws + c.ws.part);
+    a.part_bytes = static_cast<uint32_t>(c.ws.part_bytes);
+    a.tile_count = reinterpret_cast<unsigned*>(ws);
+    a.N = s.rows, a.nb = s.nb, a.row_tiles = c.row_tiles, a.tok_tiles = c.tok_tiles;
+    a.splits = c.splits, a.chunks_per_split = c.cps;
+    a.xcd_br = a.xcd_row_outer = 0;
+    if (c.splits == 1) xcd_blocks(s, c.row_tiles, c.tok_tiles, kTileM, kTileN, &a.xcd_br, &a.xcd_row_outer);
+    if (!presplit) {
+        hipLaunchKernelGGL((xsplit_kernel<QT, true>), dim3(c.npad), dim3(256), 0, stream, x, s.rows, s.K, s.nb, c.npad,
+                           reinterpret_cast<_Float16*>(ws + c.ws.xs), reinterpret_cast<float*>(ws + c.ws.bsum),
+                           reinterpret_cast<float*>(ws + c.ws.scale));
+    }
+    hipLaunchKernelGGL(kern, dim3(c.row_tiles * c.tok_tiles * c.splits), dim3(T::threads), T::lds, stream, a);
+    return hipGetLastError();
+}
+
+template <int QT>
+hipError_t launch_chunk_q(const LinearShape& s, const float* x, char* ws, hipStream_t stream, const ChunkGroup& grp,
+                          bool presplit) {
+    if (use_tile(s)) return launch_tile<QT>(s, x, ws, stream, grp, presplit);
+    const ChunkCfg c = choose_chunk(s);
+    if (c.tt == 1) return launch_chunk_t<QT, 1, 1>(s, c, x, ws, stream, grp);
+    return launch_chunk_t<QT, 2, 2>(s, c, x, ws, stream, grp);
+}
+
+// Weights start on dwords, as the tile kernel's copies and the row-pair loads need.
+bool aligned_weights(const ChunkGroup& grp) {
+    uintptr_t p = 0;
+    for (int g = 0; g < grp.n; ++g) p |= reinterpret_cast<uintptr_t>(grp.w[g]);
+    return (p & 3u) == 0;
 }
 
 bool use_chunk(const LinearShape& s, const float* x) {
-    if (!chunk_supported(s)) return false;
+    if (use_tile(s)) return static_cast<size_t>(s.M) * s.nb * block_bytes(s.qtype) < (static_cast<size_t>(1) << 32);
+    if (!chunk_supported(s) || s.rows > 128) return false;
     const ChunkCfg c = choose_chunk(s);
     const size_t wbytes = static_cast<size_t>(s.M) * s.nb * block_bytes(s.qtype);
-    return (c.xs || (reinterpret_cast<uintptr_t>(x) & 15u) == 0) && wbytes < (static_cast<size_t>(1) << 32) &&
+    return (reinterpret_cast<uintptr_t>(x) & 15u) == 0 && wbytes < (static_cast<size_t>(1) << 32) &&
            chunk_layout(s, c).part_bytes < (static_cast<size_t>(1) << 31);
 }
 
@@ -1257,25 +1259,20 @@ bool gemm_supported(const LinearShape& s) {
     return s.rows > 1 && s.nb % 2 == 0 && s.nb >= 2 && (s.qtype >= 1 && s.qtype <= 3);
 }
 
-size_t gemm_workspace_bytes(const LinearShape& s) {
-    if (!gemm_supported(s)) return 0;
-    size_t b = layout(s, choose(s)).total;
-    if (chunk_supported(s)) b = std::max(b, chunk_workspace_bytes(s));
-    return b;
-}
+size_t gemm_workspace_bytes(const LinearShape& s) { return gemm_supported(s) ? workspace_bytes(s) : 0; }
 
 hipError_t launch_gemm(const LinearShape& s, const void* w, const float* x, float* y, void* ws,
                        size_t ws_bytes, hipStream_t stream) {
     if (!gemm_supported(s)) return hipErrorNotSupported;
     if (ws == nullptr) return hipErrorInvalidValue;
     char* base = static_cast<char*>(ws);
-    if (use_chunk(s, x)) {
-        if (ws_bytes < chunk_workspace_bytes(s)) return hipErrorInvalidValue;
-        const ChunkCfg c = choose_chunk(s);
+    const ChunkGroup grp{1, {w, nullptr, nullptr}, {y, nullptr, nullptr}, {s.M, 0, 0}};
+    if (use_chunk(s, x) && (!use_tile(s) || aligned_weights(grp))) {
+        if (ws_bytes < workspace_bytes(s)) return hipErrorInvalidValue;
         switch (s.qtype) {
-            case 1: return launch_chunk_q<1>(s, c, w, x, y, base, stream);
-            case 2: return launch_chunk_q<2>(s, c, w, x, y, base, stream);
-            default: return launch_chunk_q<3>(s, c, w, x, y, base, stream);
+            case 1: return launch_chunk_q<1>(s, x, base, stream, grp, false);
+            case 2: return launch_chunk_q<2>(s, x, base, stream, grp, false);
+            default: return launch_chunk_q<3>(s, x, base, stream, grp, false);
         }
     }
     const GemmCfg c = choose(s);
@@ -1298,17 +1295,16 @@ GemmSplitX gemm_split_x(const LinearShape& s, int n, const int* M) {
         st.M += M[g];
     }
     if (!chunk_supported(st)) return r;
-    const ChunkCfg c = choose_chunk(st);
-    if (!c.xs || !use_chunk(st, nullptr)) return r;
+    if (!use_tile(st) || !use_chunk(st, nullptr)) return r;
     for (int g = 0; g + 1 < n; ++g)
-        if (M[g] % (64 * c.rw) != 0) return r;
-    const ChunkWs l = chunk_layout(st, c);
+        if (M[g] % kTileM != 0) return r;
+    const TileCfg c = choose_tile(st);
     r.ok = true;
     r.npad = c.npad;
-    r.xs = l.xs;
-    r.bsum = l.bsum;
-    r.scale = l.scale;
-    r.ws_bytes = l.total;
+    r.xs = c.ws.xs;
+    r.bsum = c.ws.bsum;
+    r.scale = c.ws.scale;
+    r.ws_bytes = workspace_bytes(st);
     return r;
 }
 
@@ -1321,7 +1317,7 @@ bool gemm_group_supported(const LinearShape& s, int n, const int* M, const float
         st.M += M[g];
     }
     if (!use_chunk(st, x)) return false;
-    const int bm = 64 * choose_chunk(st).rw;
+    const int bm = use_tile(st) ? kTileM : 64 * choose_chunk(st).rw;
     for (int g = 0; g + 1 < n; ++g)
         if (M[g] % bm != 0) return false;  // a row tile may not straddle two weights
     return true;
@@ -1337,28 +1333,31 @@ hipError_t launch_gemm_group(const LinearShape& s, int n, const void* const* w, 
         st.M += M[g];
     }
     if (!gemm_group_supported(s, n, M, x)) return hipErrorNotSupported;
-    const ChunkCfg c = choose_chunk(st);
-    if (x_split && !c.xs) return hipErrorInvalidValue;  // gemm_split_x said no
+    if (x_split && !use_tile(st)) return hipErrorInvalidValue;  // gemm_split_x said no
     if (ws == nullptr) return hipErrorInvalidValue;
-    if (ws_bytes < chunk_workspace_bytes(st)) return hipErrorInvalidValue;
+    if (ws_bytes < workspace_bytes(st)) return hipErrorInvalidValue;
     ChunkGroup grp{};
     grp.n = n;
     for (int g = 0; g < n; ++g) grp.w[g] = w[g], grp.y[g] = y[g], grp.M[g] = M[g];
+    if (use_tile(st) && !aligned_weights(grp)) return hipErrorNotSupported;
     char* base = static_cast<char*>(ws);
     switch (st.qtype) {
-        case 1: return launch_chunk_q<1>(st, c, w[0], x, y[0], base, stream, &grp, x_split);
-        case 2: return launch_chunk_q<2>(st, c, w[0], x, y[0], base, stream, &grp, x_split);
-        default: return launch_chunk_q<3>(st, c, w[0], x, y[0], base, stream, &grp, x_split);
+        case 1: return launch_chunk_q<1>(st, x, base, stream, grp, x_split);
+        case 2: return launch_chunk_q<2>(st, x, base, stream, grp, x_split);
+        default: return launch_chunk_q<3>(st, x, base, stream, grp, x_split);
     }
 }
 
 const char* gemm_kernel_name(const LinearShape& s) {
     static thread_local char buf[96];
     const char* fmt = s.qtype == 1 ? "q8_0" : s.qtype == 2 ? "q4_0" : "q4_1";
-    if (chunk_supported(s)) {
+    if (use_tile(s)) {
+        snprintf(buf, sizeof buf, "gemm_mfma_%s_tile_bm%d_bn%d_splitk%d", fmt, kTileM, kTileN, choose_tile(s).splits);
+        return buf;
+    }
+    if (chunk_supported(s) && s.rows <= 128) {
         const ChunkCfg c = choose_chunk(s);
-        snprintf(buf, sizeof buf, "gemm_mfma_%s_chunk%s_bm%d_bn%d_splitk%d", fmt, c.xs ? "_xs" : "", 64 * c.rw,
-                 16 * c.tt, c.splits);
+        snprintf(buf, sizeof buf, "gemm_mfma_%s_chunk_bm%d_bn%d_splitk%d", fmt, 64 * c.rw, 16 * c.tt, c.splits);
         return buf;
     }
     const GemmCfg c = choose(s);

@@ -23,6 +23,7 @@ namespace {
 constexpr int kXsCache = 4;
 
 typedef _Float16 xs_h8 __attribute__((ext_vector_type(8)));
+typedef _Float16 xs_h2 __attribute__((ext_vector_type(2)));
 typedef _Float16 xs_h4 __attribute__((ext_vector_type(4)));
 
 // max |x| over the workgroup (every thread gets it); `red` is 4 floats of LDS.
@@ -50,7 +51,9 @@ __device__ __forceinline__ void xsplit_scale(float mx, float& inv, float& sc) {
 // Scales, splits and stores half block hb of token row n (v: its 16
 // elements).  Called by every lane (the shuffle pairs half blocks hb and
 // hb ^ 1, held by adjacent lanes); lanes with hb >= 2 nb store nothing.
-template <int QT>
+// PACK: the block sum as the two fp16 halves of sum / 32 (|sum| <= 2^19), which
+// the large-tile GEMM multiplies on the matrix cores.
+template <int QT, bool PACK>
 __device__ __forceinline__ void xsplit_emit_half(int n, int nb, int hb, float (&v)[16], float inv,
                                                  _Float16* __restrict__ xs, float* __restrict__ bsum) {
     const bool have = hb < 2 * nb;
@@ -65,7 +68,14 @@ __device__ __forceinline__ void xsplit_emit_half(int n, int nb, int hb, float (&
     if (!have) return;
     if (half == 0) {
         // block sum in the order (elements 0..15) + (16..31), 4-element groups
-        bsum[static_cast<size_t>(n) * nb + b] = sum + other;
+        const float bs = sum + other;
+        if (PACK) {
+            const _Float16 sh = static_cast<_Float16>(bs * 0.03125f);
+            const _Float16 sl = static_cast<_Float16>(bs * 0.03125f - static_cast<float>(sh));
+            reinterpret_cast<xs_h2*>(bsum)[static_cast<size_t>(n) * nb + b] = xs_h2{sh, sl};
+        } else {
+            bsum[static_cast<size_t>(n) * nb + b] = bs;
+        }
     }
     _Float16 hi[16], lo[16];
     // hi/lo in slot order of this half block
@@ -109,7 +119,7 @@ __device__ __forceinline__ void xsplit_emit_half(int n, int nb, int hb, float (&
 // The whole split of token row n from the values the workgroup holds (thread
 // t: half blocks t + 256 c in v[c], zeros past the row; 2 nb <= 256 C):
 // the row's maximum, its scale (stored by thread 0) and every half block.
-template <int QT, int C>
+template <int QT, int C, bool PACK>
 __device__ __forceinline__ void xsplit_emit_row(int n, int nb, float (&v)[C][16], _Float16* __restrict__ xs,
                                                 float* __restrict__ bsum, float* __restrict__ scale, float* red) {
     float mx = 0.0f;
@@ -124,7 +134,7 @@ __device__ __forceinline__ void xsplit_emit_row(int n, int nb, float (&v)[C][16]
     const int iters = (2 * nb + 255) / 256;  // uniform across the workgroup
 #pragma unroll
     for (int c = 0; c < C; ++c)
-        if (c < iters) xsplit_emit_half<QT>(n, nb, static_cast<int>(threadIdx.x) + 256 * c, v[c], inv, xs, bsum);
+        if (c < iters) xsplit_emit_half<QT, PACK>(n, nb, static_cast<int>(threadIdx.x) + 256 * c, v[c], inv, xs, bsum);
 }
 
 }  // namespace

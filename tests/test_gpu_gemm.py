@@ -64,6 +64,42 @@ def test_gemm_q4_1_and_ragged(hip, orc, m, k, n):
         run(hip, orc, qt, m, k, n)
 
 
+@pytest.mark.parametrize("m,k,n", [(1, 256, 129),      # two steps of K, one row
+                                   (127, 384, 191),    # three steps (an odd count), both tile edges short
+                                   (129, 1024, 193),   # one row and one token past a tile
+                                   (128, 4096, 192),   # whole tiles, K split
+                                   (257, 11008, 256)])  # 86 steps over an uneven K split
+def test_gemm_large_tile_edges(hip, orc, m, k, n):
+    """The large-tile kernel (more than 128 token rows) at the edges of its tile
+    (128 rows x 64 tokens), of its steps (128 k) and of its K split."""
+    for fmt, qt in FMTS.items():
+        name, _ = run(hip, orc, qt, m, k, n)
+        assert "_tile_" in name, name
+
+
+def test_gemm_large_tile_needs_dword_weights(hip, orc):
+    """Weights wrapped two bytes off a dword take the general kernel instead."""
+    m, k, n = 130, 512, 150
+    rng = np.random.default_rng(31)
+    x = rng.standard_normal((n, k), dtype=np.float32)
+    xb, y = hip.DeviceBuffer.from_array(x), hip.DeviceBuffer(4 * n * m)
+    for fmt, qt in FMTS.items():
+        blocks = orc.quantize(qt, rng.standard_normal((m, k), dtype=np.float32) * np.float32(0.02), threads=THREADS)
+        buf = hip.DeviceBuffer(blocks.nbytes + 4)
+        buf.upload(blocks, 2)
+        print(f"gemm qt={qt} weights at +2 bytes", flush=True)
+
+        class At:  # the blocks inside the allocation
+            ptr, nbytes = buf.ptr + 2, blocks.nbytes
+
+        wt = hip.Weight.wrap(qt, At, blocks.shape[0], m, k)
+        wt.linear_device(xb, y, rows=n)
+        want = orc.linear(qt, x, blocks, m, threads=THREADS)
+        check_close(y.download(np.float32, n * m).reshape(n, m), want, x, qt, blocks, f"qt={qt} unaligned weights")
+        wt.free()
+        buf.free()
+
+
 def test_gemm_wide_dynamic_range(hip, orc):
     """Per-token power-of-two scaling keeps the hi/lo split exact across token
     magnitudes from 1e-6 to 1e4 (and an all-zero token)."""
