@@ -128,6 +128,14 @@ struct PickSlot {
 constexpr size_t kScratchBytes = size_t(48) << 20;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
+// Scratch of the decode attention op, one slot per stream that calls it outside
+// graph capture (the stream orders the slot's users; a recorded launch may be
+// replayed anywhere, so it gets none).  A fixed array: no allocation on any call.
+// Streams beyond the slots, and the per-thread default stream, whose one handle
+// stands for many streams, run the unsplit attention.
+constexpr int kAttnSlots = 16;
+static __device__ __align__(256) unsigned char attn_scratch[kAttnSlots][mlq::kOpAttnScratchBytes];
+
 struct DeviceState {
     std::once_flag once;
     hipError_t init_err = hipSuccess;
@@ -143,6 +151,8 @@ struct DeviceState {
     // x), so a retired buffer is kept until the process ends.
     std::vector<void*> retired_ws;
     std::vector<PickSlot> picks;
+    void* attn_scratch = nullptr;             // this device's address of `attn_scratch` (zeroed at set-up)
+    hipStream_t attn_slot[kAttnSlots] = {};  // the stream of each slot (guarded by ws_mu)
     std::mutex pin_mu;         // guards the pinned stage of file uploads
     void* pin[2] = {nullptr, nullptr};
     hipEvent_t pin_done[2] = {nullptr, nullptr};
@@ -190,6 +200,10 @@ int ensure_device(int device) {
             st.init_err = hipGetSymbolAddress(&st.scratch, HIP_SYMBOL(scratch));
         }
         if (st.init_err == hipSuccess) st.init_err = hipMemsetAsync(st.scratch, 0, kScratchBytes, st.stream);
+        if (st.init_err == hipSuccess) st.init_err = hipGetSymbolAddress(&st.attn_scratch, HIP_SYMBOL(attn_scratch));
+        if (st.init_err == hipSuccess) {
+            st.init_err = hipMemsetAsync(st.attn_scratch, 0, kAttnSlots * mlq::kOpAttnScratchBytes, st.stream);
+        }
         if (st.init_err == hipSuccess) st.init_err = hipStreamSynchronize(st.stream);
     });
     if (st.init_err != hipSuccess) return hip_fail(st.init_err, "device init");
@@ -349,6 +363,21 @@ int stream_pick(int device, hipStream_t stream, const char* caller, PickSlot* ou
     st.picks.push_back(p);
     *out = p;
     return MLQ_OK;
+}
+
+// The attention scratch of `stream`, or null (see attn_scratch).
+void* stream_attn_scratch(int device, hipStream_t stream) {
+    if (stream == hipStreamPerThread || capturing(stream)) return nullptr;
+    DeviceState& st = g_dev[device];
+    std::lock_guard<std::mutex> lock(st.ws_mu);
+    int slot = -1;
+    for (int i = 0; i < kAttnSlots && slot < 0; ++i)
+        if (st.attn_slot[i] == stream) slot = i;
+    for (int i = 0; i < kAttnSlots && slot < 0; ++i)
+        if (st.attn_slot[i] == nullptr) slot = i;
+    if (slot < 0) return nullptr;
+    st.attn_slot[slot] = stream;
+    return static_cast<char*>(st.attn_scratch) + slot * mlq::kOpAttnScratchBytes;
 }
 
 int dispatch(int device, const mlq::LinearShape& s, const void* w, const float* x, float* y,
@@ -990,6 +1019,11 @@ int mlq_hip_stream_create(int device, void** stream) {
 int mlq_hip_stream_destroy(void* stream) {
     if (stream == nullptr) return MLQ_OK;
     MLQ_HIP_CHECK(hipStreamSynchronize(static_cast<hipStream_t>(stream)));
+    for (DeviceState& st : g_dev) {  // its attention slot, idle now, is free again
+        std::lock_guard<std::mutex> lock(st.ws_mu);
+        for (hipStream_t& s : st.attn_slot)
+            if (s == static_cast<hipStream_t>(stream)) s = nullptr;
+    }
     MLQ_HIP_CHECK(hipStreamDestroy(static_cast<hipStream_t>(stream)));
     return MLQ_OK;
 }
@@ -1235,8 +1269,9 @@ int mlq_hip_attention_decode(int device, const float* q, const float* keys, cons
     if (rc == MLQ_OK) rc = check_device_ptr(values, device, caller, "value cache", cache);
     if (rc == MLQ_OK) rc = check_device_ptr(out, device, caller, "output", qb);
     if (rc != MLQ_OK) return rc;
+    const hipStream_t s = resolve_stream(device, stream);
     hipError_t e = mlq::launch_op_attention_decode(q, keys, values, layer, max_seq_len, n_heads, n_kv_heads, head_dim,
-                                                   pos, out, resolve_stream(device, stream));
+                                                   pos, out, stream_attn_scratch(device, s), s);
     return e == hipSuccess ? MLQ_OK : hip_fail(e, "op_attention_decode_kernel");
 }
 

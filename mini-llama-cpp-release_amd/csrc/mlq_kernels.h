@@ -225,6 +225,11 @@ constexpr int kOpSilu = 0;
 constexpr int kOpMul = 1;
 constexpr int kOpAdd = 2;
 constexpr int kOpAttnMaxHeadDim = 512;
+// Scratch that lets the attention split its positions over workgroups: arrival
+// counters (zero between launches), then the splits' states.  One launch at a time
+// may use it; null: one workgroup per head.
+constexpr int kOpAttnScratchGroups = 1024;
+constexpr size_t kOpAttnScratchBytes = size_t(1) << 20;
 hipError_t launch_op_rmsnorm(const float* x, const float* w, int n, float eps, float* y, hipStream_t s);
 hipError_t launch_op_elementwise(int op, const float* a, const float* b, size_t n, float* y, hipStream_t s);
 hipError_t launch_op_softmax(const float* x, int n, float* y, hipStream_t s);
@@ -232,7 +237,7 @@ hipError_t launch_op_embedding(const float* table, int dim, int token, float* y,
 hipError_t launch_op_rope(float* x, int n_heads, int head_dim, int pos, float theta, bool neox, hipStream_t s);
 hipError_t launch_op_attention_decode(const float* q, const float* keys, const float* values, int layer,
                                       int max_seq, int n_heads, int n_kv_heads, int head_dim, int pos,
-                                      float* out, hipStream_t s);
+                                      float* out, void* scratch, hipStream_t s);
 hipError_t launch_op_matmul_f32(const float* a, const float* b, int m, int k, int n, bool b_transposed, float* c,
                                 hipStream_t s);
 

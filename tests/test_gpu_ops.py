@@ -155,6 +155,88 @@ def test_attention_decode(hip, n_heads, n_kv, hd, max_seq, pos):
           f"attention {n_heads}x{hd}@{pos}")
 
 
+# (heads, kv heads, head size, position): either side of the split (49 152
+# elements of a head), short last splits and passes, groups of 1 to 12 heads (chunks
+# of 4 and 8, one short), every lane layout, a size that fills none (80), one that
+# 16-byte loads do not fit (30).
+SPLIT_SHAPES = [(4, 4, 64, 767), (4, 4, 64, 768), (2, 2, 128, 6), (2, 2, 128, 383), (2, 2, 128, 384), (8, 4, 128, 430),
+                (12, 4, 128, 777), (14, 2, 64, 1001), (12, 1, 128, 2047), (8, 2, 256, 515), (8, 1, 512, 301),
+                (6, 2, 80, 700), (64, 32, 128, 999), (6, 3, 30, 200)]
+
+
+@pytest.mark.parametrize("stream", ["library", "capture", "many"])
+def test_attention_split(hip, stream):
+    """Positions split over workgroups (the library's stream), the unsplit kernel (a
+    recorded launch, replayed, and streams past the scratch slots) and the same
+    results on all of them, call after call."""
+    layers, layer = 2, 1
+    for n_heads, n_kv, hd, pos in SPLIT_SHAPES:
+        max_seq = pos + 3
+        rng = np.random.default_rng(n_heads * 1000 + hd + pos)
+        K = rng.standard_normal((layers, max_seq, n_kv, hd)).astype(np.float32)
+        V = rng.standard_normal((layers, max_seq, n_kv, hd)).astype(np.float32)
+        q = rng.standard_normal((n_heads, hd)).astype(np.float32)
+        want = attention_ref(q, K, V, layer, pos, n_heads, n_kv, hd)
+        dq, dk, dv, o = dev(hip, q), dev(hip, K), dev(hip, V), out(hip, n_heads * hd)
+        say(f"attention {n_heads}/{n_kv} heads of {hd}, position {pos}, {stream}")
+
+        def call(s):
+            hip._check(hip.load().mlq_hip_attention_decode(0, dq.ptr, dk.ptr, dv.ptr, layers, layer, max_seq, n_heads,
+                                                            n_kv, hd, pos, o.ptr, s))
+
+        def check(what):
+            close(got(hip, o, n_heads * hd).reshape(n_heads, hd), want, f"attention {n_heads}x{hd}@{pos} {what}")
+            o.fill(0)
+
+        if stream == "library":
+            for i in range(3):
+                call(None)
+                check(f"call {i}")
+        elif stream == "capture":
+            sp = hip.stream_create(0)
+            call(sp)
+            hip.synchronize(sp)
+            check("eager")
+            g = hip.Graph.record(lambda: call(sp), sp)
+            for i in range(3):
+                g.launch(sp)
+                hip.synchronize(sp)
+                check(f"replay {i}")
+                call(sp)
+                hip.synchronize(sp)
+                check("between replays")
+            g.destroy()
+            hip.stream_destroy(sp)
+        else:
+            streams = [hip.stream_create(0) for _ in range(18)]
+            for i, sp in enumerate(streams):
+                call(sp)
+                hip.synchronize(sp)
+                check(f"stream {i}")
+            for sp in streams:
+                hip.stream_destroy(sp)
+
+
+def test_attention_split_infinities(hip):
+    """A score of -inf (a masked key) drops out of a split softmax; a NaN key makes
+    its heads NaN; an infinite v row past the position is not touched."""
+    n_heads, n_kv, hd, pos, max_seq = 4, 2, 64, 899, 902
+    rng = np.random.default_rng(5)
+    K = rng.standard_normal((1, max_seq, n_kv, hd)).astype(np.float32)
+    V = rng.standard_normal((1, max_seq, n_kv, hd)).astype(np.float32)
+    q = np.abs(rng.standard_normal((n_heads, hd))).astype(np.float32) + 0.1
+    K[0, 7, 0] = K[0, 64:96, 0] = -np.inf
+    K[0, 20, 1, 3] = np.nan
+    V[0, pos + 1:] = np.inf
+    dq, dk, dv, o = dev(hip, q), dev(hip, K), dev(hip, V), out(hip, n_heads * hd)
+    say("attention with infinities")
+    hip._check(hip.load().mlq_hip_attention_decode(0, dq.ptr, dk.ptr, dv.ptr, 1, 0, max_seq, n_heads, n_kv, hd, pos, o.ptr,
+                                                    None))
+    y = got(hip, o, n_heads * hd).reshape(n_heads, hd)
+    close(y[:2], attention_ref(q[:2], K[:, :, :1], V[:, :, :1], 0, pos, 2, 1, hd), "masked keys")
+    assert np.isnan(y[2:]).all()
+
+
 def test_attention_rejects_bad_positions(hip):
     q, kv, o = out(hip, 64), out(hip, 2 * 16 * 64), out(hip, 64)
     lib = hip.load()
