@@ -540,10 +540,10 @@ __global__ __launch_bounds__(kNormThreads) void add_rmsnorm_rows_kernel(float* _
 
 // Row kernels whose output goes straight to a prefill GEMM as its split x
 // (xsplit_device.h; the GEMM then makes no split launch of its own).
-// Workgroup `row` of 256 threads holds the row's half blocks in registers
-// (thread t: half blocks t + 256 c); rows n .. npad - 1 write a zero split
-// (the GEMM's padded token tile).  C = ceil(2 nb / 256) half blocks per
-// thread (dim = 32 nb <= 256 * 16 * kXsCache).
+// Workgroup `row` of 256 threads holds the row's items in registers (thread t:
+// items t + 256 c, two runs of four elements each); rows n .. npad - 1 write a
+// zero split (the GEMM's padded token tile).  C >= ceil(4 nb / 256) items per
+// thread (dim = 32 nb <= 256 * 8 * kXsCache).
 //
 // add_rmsnorm_rows_kernel's step for a GEMM input: X[r] += D[r] (when given),
 // then the split of rmsnorm(X[r]) * w.
@@ -558,68 +558,49 @@ __global__ __launch_bounds__(256) void add_rmsnorm_split_rows_kernel(float* __re
     const int row = blockIdx.x;
     const bool valid = row < n;
     const size_t off = static_cast<size_t>(valid ? row : 0) * dim;
-    float v[C][16], wv[C][16];
+    float v[C][8], wv[C][8], dv[C][8];
     float ss = 0.0f;
-    // Every load is unconditional (half blocks past the row re-read the last
-    // one, D absent reads X again; both are selected away): a load under a
-    // branch makes the compiler wait for it at the join, one round trip per
-    // half block.  The norm weights are requested with the row.
+    // Every load is unconditional (items past the row re-read the last one, D
+    // absent reads X again; both are selected away): a load under a branch makes
+    // the compiler wait for it at the join, one round trip per item.  The norm
+    // weights are requested with the row.
     const float* const Dp = D != nullptr ? D + off : X + off;
+    constexpr int k1 = xs_second<QT>();
+    int k0[C];
 #pragma unroll
     for (int c = 0; c < C; ++c) {
-        const int k0 = min(16 * (static_cast<int>(threadIdx.x) + 256 * c), dim - 16);
-#pragma unroll
-        for (int i = 0; i < 16; i += 4) {
-            const float4 a = *reinterpret_cast<const float4*>(w + k0 + i);
-            wv[c][i] = a.x;
-            wv[c][i + 1] = a.y;
-            wv[c][i + 2] = a.z;
-            wv[c][i + 3] = a.w;
-        }
-    }
-    float dv[C][16];
-#pragma unroll
-    for (int c = 0; c < C; ++c) {
-        const int k0 = min(16 * (static_cast<int>(threadIdx.x) + 256 * c), dim - 16);
-#pragma unroll
-        for (int i = 0; i < 16; i += 4) {
-            const float4 a = *reinterpret_cast<const float4*>(X + off + k0 + i);
-            const float4 d = *reinterpret_cast<const float4*>(Dp + k0 + i);
-            v[c][i] = a.x;
-            v[c][i + 1] = a.y;
-            v[c][i + 2] = a.z;
-            v[c][i + 3] = a.w;
-            dv[c][i] = d.x;
-            dv[c][i + 1] = d.y;
-            dv[c][i + 2] = d.z;
-            dv[c][i + 3] = d.w;
-        }
+        k0[c] = xs_first<QT>(min(static_cast<int>(threadIdx.x) + 256 * c, 4 * nb - 1));
+        xs_put4(wv[c], 0, w + k0[c]);
+        xs_put4(wv[c], 4, w + k0[c] + k1);
     }
 #pragma unroll
     for (int c = 0; c < C; ++c) {
-        const int k0 = 16 * (static_cast<int>(threadIdx.x) + 256 * c);
-        const bool in = valid && k0 < dim;
+        xs_put4(v[c], 0, X + off + k0[c]);
+        xs_put4(v[c], 4, X + off + k0[c] + k1);
+        xs_put4(dv[c], 0, Dp + k0[c]);
+        xs_put4(dv[c], 4, Dp + k0[c] + k1);
+    }
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
+    for (int c = 0; c < C; ++c) {
+        const bool in = valid && static_cast<int>(threadIdx.x) + 256 * c < 4 * nb;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
             const float a = D != nullptr ? v[c][i] + dv[c][i] : v[c][i];
             v[c][i] = in ? a : 0.0f;
             ss += v[c][i] * v[c][i];
         }
         if (in && D != nullptr) {
-#pragma unroll
-            for (int i = 0; i < 16; i += 4)
-                *reinterpret_cast<float4*>(X + off + k0 + i) =
-                    make_float4(v[c][i], v[c][i + 1], v[c][i + 2], v[c][i + 3]);
+            *reinterpret_cast<float4*>(X + off + k0[c]) = make_float4(v[c][0], v[c][1], v[c][2], v[c][3]);
+            *reinterpret_cast<float4*>(X + off + k0[c] + k1) = make_float4(v[c][4], v[c][5], v[c][6], v[c][7]);
         }
     }
     ss = wg_reduce<256, false>(ss, part);
     const float sc = 1.0f / sqrtf(ss / static_cast<float>(dim) + eps);
 #pragma unroll
     for (int c = 0; c < C; ++c) {
-        const int k0 = 16 * (static_cast<int>(threadIdx.x) + 256 * c);
-        if (valid && k0 < dim) {
+        if (valid && static_cast<int>(threadIdx.x) + 256 * c < 4 * nb) {
 #pragma unroll
-            for (int i = 0; i < 16; ++i) v[c][i] = v[c][i] * sc * wv[c][i];
+            for (int i = 0; i < 8; ++i) v[c][i] = v[c][i] * sc * wv[c][i];
         }
     }
     __syncthreads();  // part is reused by the split's maximum
@@ -636,32 +617,22 @@ __global__ __launch_bounds__(256) void swiglu_split_rows_kernel(const float* __r
     const int row = blockIdx.x;
     const bool valid = row < n;
     const size_t off = static_cast<size_t>(valid ? row : 0) * hidden;
-    float v[C][16], uv[C][16];
-    // Unconditional loads (half blocks past the row re-read the last one and
-    // are selected away), all issued before any is used.
+    float v[C][8], uv[C][8];
+    // Unconditional loads (items past the row re-read the last one and are
+    // selected away), all issued before any is used.
 #pragma unroll
     for (int c = 0; c < C; ++c) {
-        const int k0 = min(16 * (static_cast<int>(threadIdx.x) + 256 * c), hidden - 16);
-#pragma unroll
-        for (int i = 0; i < 16; i += 4) {
-            const float4 g = *reinterpret_cast<const float4*>(G + off + k0 + i);
-            const float4 u = *reinterpret_cast<const float4*>(U + off + k0 + i);
-            v[c][i] = g.x;
-            v[c][i + 1] = g.y;
-            v[c][i + 2] = g.z;
-            v[c][i + 3] = g.w;
-            uv[c][i] = u.x;
-            uv[c][i + 1] = u.y;
-            uv[c][i + 2] = u.z;
-            uv[c][i + 3] = u.w;
-        }
+        const int k0 = xs_first<QT>(min(static_cast<int>(threadIdx.x) + 256 * c, 4 * nb - 1));
+        xs_put4(v[c], 0, G + off + k0);
+        xs_put4(v[c], 4, G + off + k0 + xs_second<QT>());
+        xs_put4(uv[c], 0, U + off + k0);
+        xs_put4(uv[c], 4, U + off + k0 + xs_second<QT>());
     }
 #pragma unroll
     for (int c = 0; c < C; ++c) {
-        const int k0 = 16 * (static_cast<int>(threadIdx.x) + 256 * c);
-        const bool in = valid && k0 < hidden;
+        const bool in = valid && static_cast<int>(threadIdx.x) + 256 * c < 4 * nb;
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
+        for (int i = 0; i < 8; ++i) {
             const float gv = v[c][i];
             const float sig = 1.0f / (1.0f + expf(-gv));
             v[c][i] = in ? gv * sig * uv[c][i] : 0.0f;
@@ -1925,7 +1896,7 @@ bool Decoder::split_target(int ng, const Linear* const* w, int rows, SplitTarget
         t.w[g] = w[g]->data;
     }
     const int K = w[0]->K;
-    if (K % 32 != 0 || K > 256 * kXsCache * 16) return false;
+    if (K % 32 != 0 || K > 256 * kXsCache * 8) return false;
     t.ng = ng;
     t.shape = LinearShape{w[0]->qtype, 0, K, K / 32, rows};
     for (int g = 0; g < ng; ++g) t.shape.M += t.M[g];
@@ -1934,7 +1905,7 @@ bool Decoder::split_target(int ng, const Linear* const* w, int rows, SplitTarget
 }
 
 namespace {
-// C = half blocks per thread, from the row width (at most kXsCache).
+// C = items per thread, from the row width (at most kXsCache).
 template <int QT>
 void launch_norm_split(hipStream_t s, int npad, float* X, const float* D, const float* w, int dim, float eps, int n,
                        char* ws, const GemmSplitX& sx) {
@@ -1943,11 +1914,14 @@ void launch_norm_split(hipStream_t s, int npad, float* X, const float* D, const 
                            reinterpret_cast<_Float16*>(ws + sx.xs), reinterpret_cast<float*>(ws + sx.bsum),
                            reinterpret_cast<float*>(ws + sx.scale));
     };
-    switch ((dim / 16 + 255) / 256) {
+    switch ((dim / 8 + 255) / 256) {
         case 1: go(add_rmsnorm_split_rows_kernel<QT, 1>); break;
         case 2: go(add_rmsnorm_split_rows_kernel<QT, 2>); break;
         case 3: go(add_rmsnorm_split_rows_kernel<QT, 3>); break;
-        default: go(add_rmsnorm_split_rows_kernel<QT, 4>); break;
+        case 4: go(add_rmsnorm_split_rows_kernel<QT, 4>); break;
+        case 5:
+        case 6: go(add_rmsnorm_split_rows_kernel<QT, 6>); break;
+        default: go(add_rmsnorm_split_rows_kernel<QT, kXsCache>); break;
     }
 }
 template <int QT>
@@ -1958,11 +1932,14 @@ void launch_swiglu_split(hipStream_t s, int npad, const float* G, const float* U
                            reinterpret_cast<_Float16*>(ws + sx.xs), reinterpret_cast<float*>(ws + sx.bsum),
                            reinterpret_cast<float*>(ws + sx.scale));
     };
-    switch ((hidden / 16 + 255) / 256) {
+    switch ((hidden / 8 + 255) / 256) {
         case 1: go(swiglu_split_rows_kernel<QT, 1>); break;
         case 2: go(swiglu_split_rows_kernel<QT, 2>); break;
         case 3: go(swiglu_split_rows_kernel<QT, 3>); break;
-        default: go(swiglu_split_rows_kernel<QT, 4>); break;
+        case 4: go(swiglu_split_rows_kernel<QT, 4>); break;
+        case 5:
+        case 6: go(swiglu_split_rows_kernel<QT, 6>); break;
+        default: go(swiglu_split_rows_kernel<QT, kXsCache>); break;
     }
 }
 }  // namespace

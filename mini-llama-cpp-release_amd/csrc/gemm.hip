@@ -12,7 +12,7 @@
 //     workgroup of the split writes one contiguous row, and a GEMM chunk reads
 //     a token's four blocks as 512 contiguous bytes (against block-major
 //     storage: 4096 x 4096 Q4_0 at 512 tokens 68.3 -> 66.8 us per call).
-//  2. gemm (more than 128 tokens: the large-tile kernel of gemm_tile.h, the same
+//  2. gemm (large products: the large-tile kernel of gemm_tile.h, the same
 //     products on v_mfma_f32_32x32x16_f16): v_mfma_f32_16x16x32_f16 with A = X fragments (16 tokens x 32 k,
 //     hi then lo) and B = weight fragments (32 k x 16 weight rows) holding the
 //     block's integer codes as exact fp16 values (q, q - 8 or the Q8_0 byte).
@@ -67,74 +67,101 @@ __device__ __forceinline__ int slot_k(int g, int j) {
 }
 
 // ---------------------------------------------------------------------------
-// xsplit: one workgroup per (padded) token row; thread t takes the half blocks
-// t, t + 256, ... (16 consecutive floats each, so a wave reads 4 KB contiguous).
-// The first kXsCache of them stay in registers between the two passes (the
-// max|x| of the row, then the scaled split), so rows up to 16 384 elements are
-// read once; longer rows re-read the rest (L2 hits).  The split itself is
-// xsplit_device.h's, which kernels producing a GEMM input also use.
-template <int QT, bool PACK>
-__global__ __launch_bounds__(256) void xsplit_kernel(const float* __restrict__ x, int N, int K,
-                                                     int nb, int npad, _Float16* __restrict__ xs,
-                                                     float* __restrict__ bsum,
+// xsplit: one workgroup per (padded) token row; thread t takes the items
+// t, t + 256, ... (xsplit_device.h: two runs of four floats each).  The first
+// kXsCache of them stay in registers between the two passes (the max|x| of the
+// row, then the scaled split), so rows up to 16 384 elements are read once; longer
+// rows re-read the rest (L2 hits).  The split itself is xsplit_device.h's, which
+// kernels producing a GEMM input also use.
+template <int QT, bool PACK, int C>
+__global__ __launch_bounds__(256) void xsplit_kernel(const float* __restrict__ x, int N, int K, int nb,
+                                                     _Float16* __restrict__ xs, float* __restrict__ bsum,
                                                      float* __restrict__ scale) {
-    (void)npad;
     const int n = blockIdx.x;
     const bool valid = n < N;
     const float* xr = x + static_cast<size_t>(valid ? n : 0) * K;
     __shared__ float red[4];
-    const int nhb = 2 * nb;
+    const int items = 4 * nb;
+    const bool vec = K % 32 == 0 && (reinterpret_cast<uintptr_t>(xr) & 15u) == 0;  // K % 32: every row is like row 0
 
-    auto load16 = [&](int hb, float (&v)[16]) {
-        const int k0 = hb * 16;
-        if (!valid || hb >= nhb) {
+    auto load8 = [&](int i, float (&v)[8]) {
+        const int k0 = xs_first<QT>(i), k1 = k0 + xs_second<QT>();
+        if (!valid || i >= items) {
 #pragma unroll
-            for (int i = 0; i < 16; ++i) v[i] = 0.0f;
-        } else if (k0 + 16 <= K && (reinterpret_cast<uintptr_t>(xr + k0) & 15u) == 0) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float4 f = reinterpret_cast<const float4*>(xr + k0)[i];
-                v[4 * i] = f.x;
-                v[4 * i + 1] = f.y;
-                v[4 * i + 2] = f.z;
-                v[4 * i + 3] = f.w;
-            }
+            for (int k = 0; k < 8; ++k) v[k] = 0.0f;
         } else {
 #pragma unroll
-            for (int i = 0; i < 16; ++i) v[i] = (k0 + i < K) ? xr[k0 + i] : 0.0f;
+            for (int k = 0; k < 4; ++k) {
+                v[k] = k0 + k < K ? xr[k0 + k] : 0.0f;
+                v[4 + k] = k1 + k < K ? xr[k1 + k] : 0.0f;
+            }
         }
     };
 
-    float cache[kXsCache][16];
+    float cache[C][8];
+    if (vec) {
+        // Unconditional loads (items past the row re-read its last one): a load
+        // under a branch is waited for at the join.
 #pragma unroll
-    for (int c = 0; c < kXsCache; ++c) load16(threadIdx.x + 256 * c, cache[c]);
-    if (nhb <= 256 * kXsCache) {
-        xsplit_emit_row<QT, kXsCache, PACK>(n, nb, cache, xs, bsum, scale, red);
+        for (int c = 0; c < C; ++c) {
+            const int k0 = xs_first<QT>(min(static_cast<int>(threadIdx.x) + 256 * c, items - 1));
+            xs_put4(cache[c], 0, xr + k0);
+            xs_put4(cache[c], 4, xr + k0 + xs_second<QT>());
+        }
+#pragma unroll
+        for (int c = 0; c < C; ++c)
+            if (!valid || static_cast<int>(threadIdx.x) + 256 * c >= items) {
+#pragma unroll
+                for (int k = 0; k < 8; ++k) cache[c][k] = 0.0f;
+            }
+    } else {
+#pragma unroll
+        for (int c = 0; c < C; ++c) load8(threadIdx.x + 256 * c, cache[c]);
+    }
+    if (items <= 256 * C) {
+        xsplit_emit_row<QT, C, PACK>(n, nb, cache, xs, bsum, scale, red);
         return;
     }
     float mx = 0.0f;
 #pragma unroll
-    for (int c = 0; c < kXsCache; ++c)
+    for (int c = 0; c < C; ++c)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) mx = fmaxf(mx, fabsf(cache[c][i]));
-    for (int hb = threadIdx.x + 256 * kXsCache; hb < nhb; hb += 256) {
-        float v[16];
-        load16(hb, v);
+        for (int k = 0; k < 8; ++k) mx = fmaxf(mx, fabsf(cache[c][k]));
+    for (int i = threadIdx.x + 256 * C; i < items; i += 256) {
+        float v[8];
+        load8(i, v);
 #pragma unroll
-        for (int i = 0; i < 16; ++i) mx = fmaxf(mx, fabsf(v[i]));
+        for (int k = 0; k < 8; ++k) mx = fmaxf(mx, fabsf(v[k]));
     }
     mx = xsplit_row_max(mx, red);
     float inv, sc;
     xsplit_scale(mx, inv, sc);
     if (threadIdx.x == 0) scale[n] = sc;
-    const int iters = (nhb + 255) / 256;  // uniform across the workgroup
+    const int iters = (items + 255) / 256;  // uniform across the workgroup
 #pragma unroll
-    for (int c = 0; c < kXsCache; ++c) xsplit_emit_half<QT, PACK>(n, nb, threadIdx.x + 256 * c, cache[c], inv, xs, bsum);
-    for (int it = kXsCache; it < iters; ++it) {
-        float v[16];
-        const int hb = threadIdx.x + 256 * it;
-        load16(hb, v);
-        xsplit_emit_half<QT, PACK>(n, nb, hb, v, inv, xs, bsum);
+    for (int c = 0; c < C; ++c) xsplit_emit_item<QT, PACK>(n, nb, threadIdx.x + 256 * c, cache[c], inv, xs, bsum);
+    for (int it = C; it < iters; ++it) {
+        float v[8];
+        const int i = threadIdx.x + 256 * it;
+        load8(i, v);
+        xsplit_emit_item<QT, PACK>(n, nb, i, v, inv, xs, bsum);
+    }
+}
+
+template <int QT, bool PACK>
+void launch_xsplit(const float* x, int rows, int K, int nb, int npad, _Float16* xs, float* bsum, float* scale,
+                   hipStream_t stream) {
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(npad), dim3(256), 0, stream, x, rows, K, nb, xs, bsum, scale);
+    };
+    if (nb <= 64) {
+        go(xsplit_kernel<QT, PACK, 1>);
+    } else if (nb <= 128) {
+        go(xsplit_kernel<QT, PACK, 2>);
+    } else if (nb <= 256) {
+        go(xsplit_kernel<QT, PACK, 4>);
+    } else {
+        go(xsplit_kernel<QT, PACK, kXsCache>);
     }
 }
 
@@ -979,8 +1006,7 @@ hipError_t launch_t(const LinearShape& s, const GemmCfg& c, const WsLayout& l, c
     float* scale = reinterpret_cast<float*>(ws + l.scale);
     float* part = c.splits > 1 ? reinterpret_cast<float*>(ws + l.part) : nullptr;
     unsigned* count = reinterpret_cast<unsigned*>(ws + l.count);
-    hipLaunchKernelGGL((xsplit_kernel<QT, false>), dim3(c.npad), dim3(256), 0, stream, x, s.rows, s.K, s.nb,
-                       c.npad, xs, bsum, scale);
+    launch_xsplit<QT, false>(x, s.rows, s.K, s.nb, c.npad, xs, bsum, scale, stream);
     dim3 grid((s.M + 64 * RT - 1) / (64 * RT), c.npad / (16 * TT), c.splits);
     constexpr int lds = StreamLds<TT>::bytes;
     hipLaunchKernelGGL((gemm_stream_kernel<QT, RT, TT, (RT == 1 ? 4 : 2)>), grid, dim3(kGemmThreads), lds, stream,
@@ -1007,11 +1033,10 @@ hipError_t launch_q(const LinearShape& s, const GemmCfg& c, const WsLayout& l, c
 //    workgroup, K split until the grid is about 640 workgroups with at least
 //    4 chunks per split (fewer, longer splits beat a larger grid: the split
 //    reduction is a serial tail; short rows keep 2 chunks per split);
-//  * up to 128 tokens: 128 rows x 32 tokens; from 32 tokens on, 8 chunks per
-//    split unless the tiles alone give every CU a workgroup (then no K split).
-// More tokens run the large-tile kernel (choose_tile); for them this
-// configuration only sizes the workspace (gemm_workspace_bytes), so that the
-// shapes that fit a fixed scratch do not depend on the tile kernel's splits.
+//  * more: 128 rows x 32 tokens; 8 chunks per split unless the tiles alone give
+//    every CU a workgroup (then no K split).
+// Above 128 tokens the xs fields size the workspace only (workspace_bytes: the
+// shapes that fit a fixed scratch do not depend on which kernel runs).
 struct ChunkCfg {
     int rw, tt, row_tiles, tok_tiles, splits, cps, npad;
     bool xs;
@@ -1083,48 +1108,97 @@ size_t workspace_bytes(const LinearShape& s) {
 template <int QT> using TileShape = Tile<QT, 2, 2, 2, 1, 4, 3>;
 constexpr int kTileM = TileShape<2>::BM, kTileN = TileShape<2>::BN;
 
-struct TileCfg {
-    int row_tiles, tok_tiles, splits, cps, npad;
-    ChunkWs ws;
+// Which kernel runs a call, and with which K splits.
+struct GemmPlan {
+    bool tile = false, chunk = false;  // neither: the general kernel
+    ChunkCfg c{};                      // chunk
+    int row_tiles = 0, tok_tiles = 0, splits = 0, cps = 0, npad = 0;  // tile
+    ChunkWs ws{};
 };
 
-// K splits of the tile kernel.  One workgroup fills a CU, so the grid runs in
-// ceil(grid / 256) rounds, each about 7 us (launch or start, first copies,
-// reduction over the waves, stores) plus 1.1 us a step of 128 k; a split adds
-// about 5 us (partial tiles to memory and back).  Measured (4096 x 4096 Q4_0, us):
-// 256 tokens 35.2 / 28.1 / 39.1 with 1 / 2 / 4 splits, 512 tokens 41.5 / 59 with 1 / 2.
-TileCfg choose_tile(const LinearShape& s) {
-    TileCfg c;
-    c.row_tiles = (s.M + kTileM - 1) / kTileM;
-    c.tok_tiles = (s.rows + kTileN - 1) / kTileN;
-    c.npad = c.tok_tiles * kTileN;
-    const long long tiles = static_cast<long long>(c.row_tiles) * c.tok_tiles;
-    const int steps = s.nb / kTileBlocks;
+// The chunk kernel splits x itself, again for every row tile, and runs two
+// workgroups a CU; the tile kernel pays a launch that splits x and about 6 us a
+// round of 256 workgroups for first copies, the waves' reduction and stores, but
+// then takes half the time a step.  So small products belong to the first and large
+// ones to the second; between them the estimates below decide, fitted to (us, whole
+// calls, chunk / tile):
+//   256 x 256, 186 tokens 5.4 / 11.1;   1024 x 1024, 192 tokens 14.2 / 15.7;
+//   896 x 896, 512 tokens 12.6 / 17.4;  2048 x 2048, 192 tokens 17.5 / 20.6;
+//   4096 x 4096, 64 / 96 / 192 / 512 tokens 18.5 / 21.1, 24.0 / 25.1, 39.6 / 29.8, 69.5 / 42.3;
+//   11008 x 4096, 64 / 128 tokens 36.1 / 27.6, 67.8 / 37.7;  4096 x 11008 Q8_0, 64 tokens 49.9 / 31.4.
+// A step (128 k) of a tile round takes 0.62 us plus 0.0018 us a workgroup of the
+// round (Q8_0 and Q4_1 an eighth more), a chunk step 1.25 us with one workgroup a CU
+// and 2 with two; K splits cost 2 + 0.6 us a split (tile) or 4.5 us.
+double tile_us(const LinearShape& s, long long grid, int cps, int splits, bool split_x, int npad) {
+    const double f = s.qtype == 2 ? 1.0 : 1.125;
+    auto round = [&](double wgs) { return 6.0 + f * (0.62 + 0.0018 * wgs) * cps; };
+    double us = static_cast<double>(grid / 256) * round(256.0);
+    if (grid % 256 != 0) us += round(static_cast<double>(grid % 256));
+    if (splits > 1) us += 2.0 + 0.6 * splits;
+    if (split_x) us += 4.0 + 1.5e-6 * npad * s.K;
+    return us;
+}
+
+double chunk_us(long long grid, int cps, int splits) {
+    double us = static_cast<double>(grid / 512) * (3.5 + 2.0 * cps);
+    const long long rest = grid % 512;
+    if (rest > 0) us += 3.5 + (rest <= 256 ? 1.25 : 2.0) * cps;
+    return us + (splits > 1 ? 4.5 : 0.0);
+}
+
+// presplit: x's producer writes the split x (tile kernel only; no split launch).
+GemmPlan choose_plan(const LinearShape& s, bool x_aligned, bool presplit) {
+    GemmPlan p;
+    if (!chunk_supported(s) || static_cast<size_t>(s.M) * s.nb * block_bytes(s.qtype) >= (static_cast<size_t>(1) << 32)) return p;
     const size_t most = workspace_bytes(s);
-    c.splits = 0;
+    const int steps = s.nb / kTileBlocks;
     double best = 0.0;
+    if (x_aligned) {
+        ChunkCfg c = choose_chunk(s);
+        if (c.xs) {
+            c.xs = false;
+            c.tt = 2;
+            c.tok_tiles = (s.rows + 31) / 32;
+            c.npad = 32 * c.tok_tiles;
+            const long long tiles = static_cast<long long>(c.row_tiles) * c.tok_tiles;
+            c.splits = tiles >= 256 ? 1 : std::max(1, steps / 8);
+            c.cps = (steps + c.splits - 1) / c.splits;
+            c.splits = (steps + c.cps - 1) / c.cps;
+            if (c.splits > 1 && chunk_layout(s, c).total > most) c.splits = 1, c.cps = steps;
+        }
+        const long long grid = static_cast<long long>(c.row_tiles) * c.tok_tiles * c.splits;
+        if (chunk_layout(s, c).part_bytes < (static_cast<size_t>(1) << 31)) {
+            p.chunk = true;
+            p.c = c;
+            best = chunk_us(grid, c.cps, c.splits);
+            if (s.rows <= 16) return p;  // a quarter of a tile's tokens
+        }
+    }
+    if (static_cast<size_t>(s.nb) * kTileN * 128 >= (static_cast<size_t>(1) << 31)) return p;
+    p.row_tiles = (s.M + kTileM - 1) / kTileM;
+    p.tok_tiles = (s.rows + kTileN - 1) / kTileN;
+    p.npad = p.tok_tiles * kTileN;
+    const long long tiles = static_cast<long long>(p.row_tiles) * p.tok_tiles;
     for (int want = 1; want <= 16 && want <= steps; ++want) {
         const int cps = (steps + want - 1) / want;
         const int splits = (steps + cps - 1) / cps;
         if (splits != want || (splits > 1 && (cps < 4 || tiles > kGemmMaxTiles))) continue;
         const size_t part = splits == 1 ? 0 : static_cast<size_t>(tiles) * splits * (kTileM * kTileN * 4);
-        const ChunkWs ws = ws_layout(s, true, c.npad, part);
-        if (splits > 1 && (ws.total > most || part >= (static_cast<size_t>(1) << 31))) continue;
-        const double rounds = static_cast<double>((tiles * splits + 255) / 256);
-        const double us = rounds * (7.0 + 1.1 * cps) + (splits > 1 ? 5.0 : 0.0);
-        if (c.splits == 0 || us < best) {
-            best = us;
-            c.splits = splits;
-            c.cps = cps;
-            c.ws = ws;
-        }
+        const ChunkWs ws = ws_layout(s, true, p.npad, part);
+        if (ws.total > most || part >= (static_cast<size_t>(1) << 31)) continue;
+        const double us = tile_us(s, tiles * splits, cps, splits, !presplit, p.npad);
+        if ((p.tile || p.chunk) && us >= best) continue;
+        best = us;
+        p.tile = true;
+        p.chunk = false;
+        p.splits = splits;
+        p.cps = cps;
+        p.ws = ws;
     }
-    return c;
+    return p;
 }
 
-bool use_tile(const LinearShape& s) {
-    return chunk_supported(s) && s.rows > 128 && static_cast<size_t>(s.nb) * kTileN * 128 < (static_cast<size_t>(1) << 31);
-}
+bool x_on_16(const float* x) { return (reinterpret_cast<uintptr_t>(x) & 15u) == 0; }
 
 // Weights of a grouped call: n <= 3 linears with the same qtype, K and rows.
 struct ChunkGroup {
@@ -1190,8 +1264,8 @@ hipError_t launch_chunk_t(const LinearShape& s, const ChunkCfg& c, const float* 
 }
 
 template <int QT>
-hipError_t launch_tile(const LinearShape& s, const float* x, char* ws, hipStream_t stream, const ChunkGroup& grp,
-                       bool presplit) {
+hipError_t launch_tile(const LinearShape& s, const GemmPlan& c, const float* x, char* ws, hipStream_t stream,
+                       const ChunkGroup& grp, bool presplit) {
     using T = TileShape<QT>;
     static_assert(T::BM == kTileM && T::BN == kTileN && T::lds <= 160 * 1024 - 16, "tile");
     auto kern = gemm_tile_kernel<QT, 2, 2, 2, 1, 4, 3>;
@@ -1200,7 +1274,6 @@ hipError_t launch_tile(const LinearShape& s, const float* x, char* ws, hipStream
                                    T::lds) == hipSuccess;
     }();
     if (!attr) return hipErrorInvalidConfiguration;
-    const TileCfg c = choose_tile(s);
     TileArgs a;
     for (int g = 0; g < 3; ++g) {
         a.W[g] = static_cast<const uint8_t*>(grp.w[g]);
@@ -1220,37 +1293,35 @@ hipError_t launch_tile(const LinearShape& s, const float* x, char* ws, hipStream
     a.xcd_br = a.xcd_row_outer = 0;
     if (c.splits == 1) xcd_blocks(s, c.row_tiles, c.tok_tiles, kTileM, kTileN, &a.xcd_br, &a.xcd_row_outer);
     if (!presplit) {
-        hipLaunchKernelGGL((xsplit_kernel<QT, true>), dim3(c.npad), dim3(256), 0, stream, x, s.rows, s.K, s.nb, c.npad,
-                           reinterpret_cast<_Float16*>(ws + c.ws.xs), reinterpret_cast<float*>(ws + c.ws.bsum),
-                           reinterpret_cast<float*>(ws + c.ws.scale));
+        launch_xsplit<QT, true>(x, s.rows, s.K, s.nb, c.npad, reinterpret_cast<_Float16*>(ws + c.ws.xs),
+                                reinterpret_cast<float*>(ws + c.ws.bsum), reinterpret_cast<float*>(ws + c.ws.scale), stream);
     }
     hipLaunchKernelGGL(kern, dim3(c.row_tiles * c.tok_tiles * c.splits), dim3(T::threads), T::lds, stream, a);
     return hipGetLastError();
 }
 
 template <int QT>
-hipError_t launch_chunk_q(const LinearShape& s, const float* x, char* ws, hipStream_t stream, const ChunkGroup& grp,
-                          bool presplit) {
-    if (use_tile(s)) return launch_tile<QT>(s, x, ws, stream, grp, presplit);
-    const ChunkCfg c = choose_chunk(s);
-    if (c.tt == 1) return launch_chunk_t<QT, 1, 1>(s, c, x, ws, stream, grp);
-    return launch_chunk_t<QT, 2, 2>(s, c, x, ws, stream, grp);
+hipError_t launch_plan(const LinearShape& s, const GemmPlan& p, const float* x, char* ws, hipStream_t stream,
+                       const ChunkGroup& grp, bool presplit) {
+    if (p.tile) return launch_tile<QT>(s, p, x, ws, stream, grp, presplit);
+    if (p.c.tt == 1) return launch_chunk_t<QT, 1, 1>(s, p.c, x, ws, stream, grp);
+    return launch_chunk_t<QT, 2, 2>(s, p.c, x, ws, stream, grp);
 }
 
-// Weights start on dwords, as the tile kernel's copies and the row-pair loads need.
+hipError_t launch_plan(const LinearShape& s, const GemmPlan& p, const float* x, char* ws, hipStream_t stream,
+                       const ChunkGroup& grp, bool presplit) {
+    switch (s.qtype) {
+        case 1: return launch_plan<1>(s, p, x, ws, stream, grp, presplit);
+        case 2: return launch_plan<2>(s, p, x, ws, stream, grp, presplit);
+        default: return launch_plan<3>(s, p, x, ws, stream, grp, presplit);
+    }
+}
+
+// The tile kernel's copies take weights that start on a dword.
 bool aligned_weights(const ChunkGroup& grp) {
     uintptr_t p = 0;
     for (int g = 0; g < grp.n; ++g) p |= reinterpret_cast<uintptr_t>(grp.w[g]);
     return (p & 3u) == 0;
-}
-
-bool use_chunk(const LinearShape& s, const float* x) {
-    if (use_tile(s)) return static_cast<size_t>(s.M) * s.nb * block_bytes(s.qtype) < (static_cast<size_t>(1) << 32);
-    if (!chunk_supported(s) || s.rows > 128) return false;
-    const ChunkCfg c = choose_chunk(s);
-    const size_t wbytes = static_cast<size_t>(s.M) * s.nb * block_bytes(s.qtype);
-    return (reinterpret_cast<uintptr_t>(x) & 15u) == 0 && wbytes < (static_cast<size_t>(1) << 32) &&
-           chunk_layout(s, c).part_bytes < (static_cast<size_t>(1) << 31);
 }
 
 }  // namespace
@@ -1267,13 +1338,10 @@ hipError_t launch_gemm(const LinearShape& s, const void* w, const float* x, floa
     if (ws == nullptr) return hipErrorInvalidValue;
     char* base = static_cast<char*>(ws);
     const ChunkGroup grp{1, {w, nullptr, nullptr}, {y, nullptr, nullptr}, {s.M, 0, 0}};
-    if (use_chunk(s, x) && (!use_tile(s) || aligned_weights(grp))) {
+    const GemmPlan p = choose_plan(s, x_on_16(x), false);
+    if (p.chunk || (p.tile && aligned_weights(grp))) {
         if (ws_bytes < workspace_bytes(s)) return hipErrorInvalidValue;
-        switch (s.qtype) {
-            case 1: return launch_chunk_q<1>(s, x, base, stream, grp, false);
-            case 2: return launch_chunk_q<2>(s, x, base, stream, grp, false);
-            default: return launch_chunk_q<3>(s, x, base, stream, grp, false);
-        }
+        return launch_plan(s, p, x, base, stream, grp, false);
     }
     const GemmCfg c = choose(s);
     const WsLayout l = layout(s, c);
@@ -1295,10 +1363,10 @@ GemmSplitX gemm_split_x(const LinearShape& s, int n, const int* M) {
         st.M += M[g];
     }
     if (!chunk_supported(st)) return r;
-    if (!use_tile(st) || !use_chunk(st, nullptr)) return r;
+    const GemmPlan c = choose_plan(st, true, true);
+    if (!c.tile) return r;
     for (int g = 0; g + 1 < n; ++g)
         if (M[g] % kTileM != 0) return r;
-    const TileCfg c = choose_tile(st);
     r.ok = true;
     r.npad = c.npad;
     r.xs = c.ws.xs;
@@ -1316,8 +1384,9 @@ bool gemm_group_supported(const LinearShape& s, int n, const int* M, const float
         if (M[g] <= 0) return false;
         st.M += M[g];
     }
-    if (!use_chunk(st, x)) return false;
-    const int bm = use_tile(st) ? kTileM : 64 * choose_chunk(st).rw;
+    const GemmPlan p = choose_plan(st, x_on_16(x), false);
+    if (!p.tile && !p.chunk) return false;
+    const int bm = p.tile ? kTileM : 64 * p.c.rw;
     for (int g = 0; g + 1 < n; ++g)
         if (M[g] % bm != 0) return false;  // a row tile may not straddle two weights
     return true;
@@ -1332,32 +1401,28 @@ hipError_t launch_gemm_group(const LinearShape& s, int n, const void* const* w, 
         if (M[g] <= 0) return hipErrorInvalidValue;
         st.M += M[g];
     }
-    if (!gemm_group_supported(s, n, M, x)) return hipErrorNotSupported;
-    if (x_split && !use_tile(st)) return hipErrorInvalidValue;  // gemm_split_x said no
+    if (!x_split && !gemm_group_supported(s, n, M, x)) return hipErrorNotSupported;
+    const GemmPlan p = choose_plan(st, x_on_16(x), x_split);
+    if (x_split && !p.tile) return hipErrorInvalidValue;  // gemm_split_x said no
     if (ws == nullptr) return hipErrorInvalidValue;
     if (ws_bytes < workspace_bytes(st)) return hipErrorInvalidValue;
     ChunkGroup grp{};
     grp.n = n;
     for (int g = 0; g < n; ++g) grp.w[g] = w[g], grp.y[g] = y[g], grp.M[g] = M[g];
-    if (use_tile(st) && !aligned_weights(grp)) return hipErrorNotSupported;
-    char* base = static_cast<char*>(ws);
-    switch (st.qtype) {
-        case 1: return launch_chunk_q<1>(st, x, base, stream, grp, x_split);
-        case 2: return launch_chunk_q<2>(st, x, base, stream, grp, x_split);
-        default: return launch_chunk_q<3>(st, x, base, stream, grp, x_split);
-    }
+    if (p.tile && !aligned_weights(grp)) return hipErrorNotSupported;
+    return launch_plan(st, p, x, static_cast<char*>(ws), stream, grp, x_split);
 }
 
 const char* gemm_kernel_name(const LinearShape& s) {
     static thread_local char buf[96];
     const char* fmt = s.qtype == 1 ? "q8_0" : s.qtype == 2 ? "q4_0" : "q4_1";
-    if (use_tile(s)) {
-        snprintf(buf, sizeof buf, "gemm_mfma_%s_tile_bm%d_bn%d_splitk%d", fmt, kTileM, kTileN, choose_tile(s).splits);
+    const GemmPlan p = choose_plan(s, true, false);
+    if (p.tile) {
+        snprintf(buf, sizeof buf, "gemm_mfma_%s_tile_bm%d_bn%d_splitk%d", fmt, kTileM, kTileN, p.splits);
         return buf;
     }
-    if (chunk_supported(s) && s.rows <= 128) {
-        const ChunkCfg c = choose_chunk(s);
-        snprintf(buf, sizeof buf, "gemm_mfma_%s_chunk_bm%d_bn%d_splitk%d", fmt, 64 * c.rw, 16 * c.tt, c.splits);
+    if (p.chunk) {
+        snprintf(buf, sizeof buf, "gemm_mfma_%s_chunk_bm%d_bn%d_splitk%d", fmt, 64 * p.c.rw, 16 * p.c.tt, p.c.splits);
         return buf;
     }
     const GemmCfg c = choose(s);

@@ -1,5 +1,5 @@
-// Large-tile MFMA kernel of the batched GEMM, for more than 128 token rows
-// (included by gemm.hip, whose header gives the arithmetic: x split once into
+// Large-tile MFMA kernel of the batched GEMM (included by gemm.hip, whose
+// choose_plan says which calls it takes and whose header gives the arithmetic: x split once into
 // fp16 hi + lo per token, weights as exact fp16 integers, one block of 32 k folded
 // into the f32 sums at a time with its scale).
 //

@@ -17,10 +17,24 @@
 namespace mlq {
 namespace {
 
-// Half blocks (16 elements) a thread holds: thread t holds half blocks
-// t + 256 c, c < kXsCache, so rows of up to 16 384 elements are split from
-// registers.
-constexpr int kXsCache = 4;
+// An item is the eight elements of one fragment slot run: item i is slots
+// 8 g .. 8 g + 7 of block i / 4, g = i % 4, so it leaves as one 16-byte hi and one
+// 16-byte lo store, the four items of a block side by side.  (Sixteen consecutive
+// elements per thread, the earlier split, left in 8-byte pieces 16 bytes apart: the
+// split of 512 x 4096 took 9 us of the GEMM call, now 7.)
+// Thread t holds items t + 256 c, c < kXsCache, so rows of up to 16 384 elements
+// are split from registers.
+constexpr int kXsCache = 8;
+
+// First element of item i's two runs of four.
+template <int QT>
+__device__ __forceinline__ int xs_first(int i) {
+    return 32 * (i >> 2) + (QT == 1 ? 8 : 4) * (i & 3);
+}
+template <int QT>
+__device__ __forceinline__ constexpr int xs_second() {
+    return QT == 1 ? 4 : 16;  // from the first run
+}
 
 typedef _Float16 xs_h8 __attribute__((ext_vector_type(8)));
 typedef _Float16 xs_h2 __attribute__((ext_vector_type(2)));
@@ -48,93 +62,71 @@ __device__ __forceinline__ void xsplit_scale(float mx, float& inv, float& sc) {
     }
 }
 
-// Scales, splits and stores half block hb of token row n (v: its 16
-// elements).  Called by every lane (the shuffle pairs half blocks hb and
-// hb ^ 1, held by adjacent lanes); lanes with hb >= 2 nb store nothing.
+// Scales, splits and stores item i of token row n (v: its two runs).  Called by
+// every lane (a block's four items are on adjacent lanes); items past the row
+// store nothing.
 // PACK: the block sum as the two fp16 halves of sum / 32 (|sum| <= 2^19), which
 // the large-tile GEMM multiplies on the matrix cores.
 template <int QT, bool PACK>
-__device__ __forceinline__ void xsplit_emit_half(int n, int nb, int hb, float (&v)[16], float inv,
+__device__ __forceinline__ void xsplit_emit_item(int n, int nb, int i, float (&v)[8], float inv,
                                                  _Float16* __restrict__ xs, float* __restrict__ bsum) {
-    const bool have = hb < 2 * nb;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) v[i] *= inv;
-    float sum = 0.0f;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) sum += (v[4 * q] + v[4 * q + 1]) + (v[4 * q + 2] + v[4 * q + 3]);
-    const float other = __shfl_xor(sum, 1, 64);
-    const int b = hb >> 1;
-    const int half = hb & 1;
-    if (!have) return;
-    if (half == 0) {
-        // block sum in the order (elements 0..15) + (16..31), 4-element groups
-        const float bs = sum + other;
+    for (int k = 0; k < 8; ++k) v[k] *= inv;
+    float sum = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+    auto add_lane = [](float s, int other) { return s + __builtin_bit_cast(float, other); };
+    sum = add_lane(sum, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, sum), 0xB1, 0xF, 0xF, true));  // lane ^ 1
+    sum = add_lane(sum, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, sum), 0x4E, 0xF, 0xF, true));  // lane ^ 2
+    if (i >= 4 * nb) return;
+    const int g = i & 3;
+    const size_t b = static_cast<size_t>(n) * nb + (i >> 2);
+    if (g == 0) {
         if (PACK) {
-            const _Float16 sh = static_cast<_Float16>(bs * 0.03125f);
-            const _Float16 sl = static_cast<_Float16>(bs * 0.03125f - static_cast<float>(sh));
-            reinterpret_cast<xs_h2*>(bsum)[static_cast<size_t>(n) * nb + b] = xs_h2{sh, sl};
+            const _Float16 sh = static_cast<_Float16>(sum * 0.03125f);
+            const _Float16 sl = static_cast<_Float16>(sum * 0.03125f - static_cast<float>(sh));
+            reinterpret_cast<xs_h2*>(bsum)[b] = xs_h2{sh, sl};
         } else {
-            bsum[static_cast<size_t>(n) * nb + b] = bs;
+            bsum[b] = sum;
         }
     }
-    _Float16 hi[16], lo[16];
-    // hi/lo in slot order of this half block
+    xs_h8 hi, lo;
 #pragma unroll
-    for (int j = 0; j < 16; ++j) {
-        int e;  // element (0..15 within the half) that lands in the j-th slot of the half
-        if (QT == 1) {
-            e = j;
-        } else {
-            const int t = j & 3;
-            e = 4 * (j >> 2) + ((t == 1) ? 2 : (t == 2) ? 1 : t);
-        }
-        const float f = v[e];
-        const _Float16 h = static_cast<_Float16>(f);
+    for (int j = 0; j < 8; ++j) {
+        // Q4 fragments take each run as elements 0, 2, 1, 3.
+        const int k = QT == 1 ? j : (j & 4) + (((j & 1) << 1) | ((j >> 1) & 1));
+        const _Float16 h = static_cast<_Float16>(v[k]);
         hi[j] = h;
-        lo[j] = static_cast<_Float16>(f - static_cast<float>(h));
+        lo[j] = static_cast<_Float16>(v[k] - static_cast<float>(h));
     }
-    _Float16* dst = xs + (static_cast<size_t>(n) * nb + b) * 64;
-    if (QT == 1) {
-        // slots 16*half .. +15 (two 16-byte chunks) for hi, +32 for lo
-#pragma unroll
-        for (int c = 0; c < 2; ++c) {
-            *reinterpret_cast<xs_h8*>(dst + 16 * half + 8 * c) =
-                xs_h8{hi[8 * c], hi[8 * c + 1], hi[8 * c + 2], hi[8 * c + 3], hi[8 * c + 4], hi[8 * c + 5],
-                      hi[8 * c + 6], hi[8 * c + 7]};
-            *reinterpret_cast<xs_h8*>(dst + 32 + 16 * half + 8 * c) =
-                xs_h8{lo[8 * c], lo[8 * c + 1], lo[8 * c + 2], lo[8 * c + 3], lo[8 * c + 4], lo[8 * c + 5],
-                      lo[8 * c + 6], lo[8 * c + 7]};
-        }
-    } else {
-        // group g's slots 8g + 4*half .. +3 hold this half's elements 4g .. 4g+3
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            *reinterpret_cast<xs_h4*>(dst + 8 * g + 4 * half) = xs_h4{hi[4 * g], hi[4 * g + 1], hi[4 * g + 2], hi[4 * g + 3]};
-            *reinterpret_cast<xs_h4*>(dst + 32 + 8 * g + 4 * half) =
-                xs_h4{lo[4 * g], lo[4 * g + 1], lo[4 * g + 2], lo[4 * g + 3]};
-        }
-    }
+    _Float16* dst = xs + b * 64 + 8 * g;
+    *reinterpret_cast<xs_h8*>(dst) = hi;
+    *reinterpret_cast<xs_h8*>(dst + 32) = lo;
 }
 
 // The whole split of token row n from the values the workgroup holds (thread
-// t: half blocks t + 256 c in v[c], zeros past the row; 2 nb <= 256 C):
-// the row's maximum, its scale (stored by thread 0) and every half block.
+// t: items t + 256 c in v[c], zeros past the row; 4 nb <= 256 C): the row's
+// maximum, its scale (stored by thread 0) and every item.
 template <int QT, int C, bool PACK>
-__device__ __forceinline__ void xsplit_emit_row(int n, int nb, float (&v)[C][16], _Float16* __restrict__ xs,
+__device__ __forceinline__ void xsplit_emit_row(int n, int nb, float (&v)[C][8], _Float16* __restrict__ xs,
                                                 float* __restrict__ bsum, float* __restrict__ scale, float* red) {
     float mx = 0.0f;
 #pragma unroll
     for (int c = 0; c < C; ++c)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) mx = fmaxf(mx, fabsf(v[c][i]));
+        for (int i = 0; i < 8; ++i) mx = fmaxf(mx, fabsf(v[c][i]));
     mx = xsplit_row_max(mx, red);
     float inv, sc;
     xsplit_scale(mx, inv, sc);
     if (threadIdx.x == 0) scale[n] = sc;
-    const int iters = (2 * nb + 255) / 256;  // uniform across the workgroup
+    const int iters = (4 * nb + 255) / 256;  // uniform across the workgroup
 #pragma unroll
     for (int c = 0; c < C; ++c)
-        if (c < iters) xsplit_emit_half<QT, PACK>(n, nb, static_cast<int>(threadIdx.x) + 256 * c, v[c], inv, xs, bsum);
+        if (c < iters) xsplit_emit_item<QT, PACK>(n, nb, static_cast<int>(threadIdx.x) + 256 * c, v[c], inv, xs, bsum);
+}
+
+// One float4 of `p` into v[k .. k + 3].
+__device__ __forceinline__ void xs_put4(float (&v)[8], int k, const float* p) {
+    const float4 f = *reinterpret_cast<const float4*>(p);
+    v[k] = f.x, v[k + 1] = f.y, v[k + 2] = f.z, v[k + 3] = f.w;
 }
 
 }  // namespace

@@ -64,26 +64,35 @@ def test_gemm_q4_1_and_ragged(hip, orc, m, k, n):
         run(hip, orc, qt, m, k, n)
 
 
-@pytest.mark.parametrize("m,k,n", [(1, 256, 129),      # two steps of K, one row
-                                   (127, 384, 191),    # three steps (an odd count), both tile edges short
-                                   (129, 1024, 193),   # one row and one token past a tile
-                                   (128, 4096, 192),   # whole tiles, K split
-                                   (257, 11008, 256)])  # 86 steps over an uneven K split
+@pytest.mark.parametrize("m,k,n", [(4097, 1664, 333),   # 13 steps (an odd count), one row and 13 tokens past a tile
+                                   (3999, 2048, 257),   # short last row tile, one token past a tile
+                                   (4097, 4096, 129),   # two K splits
+                                   (11009, 4096, 65),   # below the chunk kernel's old limit of 128 tokens
+                                   (4095, 11008, 64)])  # 86 steps over eight uneven K splits
 def test_gemm_large_tile_edges(hip, orc, m, k, n):
-    """The large-tile kernel (more than 128 token rows) at the edges of its tile
-    (128 rows x 64 tokens), of its steps (128 k) and of its K split."""
+    """The large-tile kernel at the edges of its tile (128 rows x 64 tokens), of its
+    steps (128 k) and of its K split."""
     for fmt, qt in FMTS.items():
         name, _ = run(hip, orc, qt, m, k, n)
         assert "_tile_" in name, name
 
 
+@pytest.mark.parametrize("m,k,n", [(1, 256, 129), (257, 11008, 256), (2048, 2048, 192), (129, 1024, 1030)])
+def test_gemm_chunk_above_128_tokens(hip, orc, m, k, n):
+    """Small products above 128 token rows: the chunk kernel, x split in it."""
+    for fmt, qt in FMTS.items():
+        name, _ = run(hip, orc, qt, m, k, n)
+        assert "_chunk_" in name, name
+
+
 def test_gemm_large_tile_needs_dword_weights(hip, orc):
     """Weights wrapped two bytes off a dword take the general kernel instead."""
-    m, k, n = 130, 512, 150
+    m, k, n = 4097, 1664, 333
     rng = np.random.default_rng(31)
     x = rng.standard_normal((n, k), dtype=np.float32)
     xb, y = hip.DeviceBuffer.from_array(x), hip.DeviceBuffer(4 * n * m)
     for fmt, qt in FMTS.items():
+        assert "_tile_" in hip.kernel_name(qt, n, m, k)
         blocks = orc.quantize(qt, rng.standard_normal((m, k), dtype=np.float32) * np.float32(0.02), threads=THREADS)
         buf = hip.DeviceBuffer(blocks.nbytes + 4)
         buf.upload(blocks, 2)
