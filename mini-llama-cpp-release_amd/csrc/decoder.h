@@ -126,6 +126,8 @@ private:
     bool prefill_batched() const;
     void ensure_prefill();
     void ensure_io(size_t need);
+    void set_state(const DecodeState& st, const int* tokens, int n);
+    void finish(float* logits_host);
 
     DecoderConfig cfg_;
     int device_ = 0;
@@ -146,6 +148,10 @@ private:
     int32_t* io_ = nullptr;      // prompt tokens then generated tokens
     size_t io_cap_ = 0;
     void* pick_ = nullptr;       // PickState
+    // Pinned host memory of the synchronous calls: [DecodeState][logits][prompt tokens].
+    static constexpr size_t kHostLogitsAt = 256;
+    void* host_ = nullptr;
+    size_t host_tokens_at_ = 0;
     float* attn_part_ = nullptr;     // [n_heads][attn_splits_][head_dim + 2]: split attention states
     unsigned* attn_cnt_ = nullptr;   // [n_heads] arrival counts of the split attention
     int attn_splits_ = 1;

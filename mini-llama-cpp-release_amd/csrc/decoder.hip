@@ -58,6 +58,28 @@ __device__ __forceinline__ float wg_reduce(float v, float* part) {
     return r;
 }
 
+// The state of a synchronous call, from launch arguments: a copy from pageable host
+// memory would be staged by the runtime ahead of the step.
+// A prompt's tokens come from pinned host memory, read once here (the embedding's
+// many workgroups reading them from there cost 50 us at 300 tokens).
+__global__ __launch_bounds__(1024) void set_state_kernel(DecodeState* st, DecodeState v, const int32_t* __restrict__ tokens,
+                                                         int n, int32_t* __restrict__ io) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) *st = v;
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) io[i] = tokens[i];
+}
+
+// The results of a synchronous call into pinned host memory: the state, then the
+// logits (when wanted).  The two copies to pageable memory this replaces cost the
+// host about 40 us a call (a 2-layer model's step at 700 positions 161 -> 122 us).
+__global__ __launch_bounds__(256) void publish_kernel(const DecodeState* st, const float* __restrict__ logits, int n,
+                                                      DecodeState* __restrict__ st_out, float* __restrict__ out) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) *st_out = *st;
+    const int n4 = n / 4;
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n4; i += gridDim.x * blockDim.x)
+        reinterpret_cast<float4*>(out)[i] = reinterpret_cast<const float4*>(logits)[i];
+    if (blockIdx.x == 0 && static_cast<int>(threadIdx.x) < n % 4) out[4 * n4 + threadIdx.x] = logits[4 * n4 + threadIdx.x];
+}
+
 // x[dim] = embedding[token] (embed_token, src/forward.cpp:496-503).  A token
 // out of range flags the step and reads row 0.
 __global__ __launch_bounds__(256) void embed_kernel(const float* __restrict__ emb, int vocab, int dim,
@@ -488,15 +510,36 @@ __global__ __launch_bounds__(kFlashThreads) void attention_rope_kernel(
     __syncthreads();
     if (last_in == 0u || tid >= HD) return;
     const float* ph = part + static_cast<size_t>(h) * nsplit * (HD + 2);
+    // Eight splits' words in flight at a time: one trip to the point of coherence
+    // a batch (a load per split in a plain loop was a trip each, twice: 7 us of the
+    // launch at 700 positions, six splits).
+    constexpr int U = 8;
     float mx = -INFINITY;
-    for (int j = 0; j < S; ++j) mx = fmaxf(mx, __hip_atomic_load(ph + j * (HD + 2), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
     float num = 0.0f;
     float den = 0.0f;
-    for (int j = 0; j < S; ++j) {
-        const float* pj = ph + j * (HD + 2);
-        const float w = expf(__hip_atomic_load(pj, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - mx);
-        den += w * __hip_atomic_load(pj + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        num += w * __hip_atomic_load(pj + 2 + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int j0 = 0; j0 < S; j0 += U) {
+        float mj[U], lj[U], nj[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const float* pj = ph + min(j0 + u, S - 1) * (HD + 2);
+            mj[u] = __hip_atomic_load(pj, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            lj[u] = __hip_atomic_load(pj + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            nj[u] = __hip_atomic_load(pj + 2 + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        float mn = mx;
+#pragma unroll
+        for (int u = 0; u < U; ++u) mn = fmaxf(mn, mj[u]);
+        const float f = j0 == 0 ? 0.0f : expf(mx - mn);
+        num = j0 == 0 ? 0.0f : num * f;
+        den = j0 == 0 ? 0.0f : den * f;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (j0 + u >= S) continue;
+            const float w = expf(mj[u] - mn);
+            den += w * lj[u];
+            num += w * nj[u];
+        }
+        mx = mn;
     }
     out[h * HD + tid] = num / den;
 }
@@ -1560,6 +1603,10 @@ std::unique_ptr<Decoder> Decoder::from_gguf(const std::string& path, int device,
     d->attn_part_ = f32buf(static_cast<size_t>(c.n_heads) * d->attn_splits_ * (c.head_dim + 2));
     d->attn_cnt_ = static_cast<unsigned*>(alloc(static_cast<size_t>(c.n_heads) * sizeof(unsigned)));
     d->check(hipMemset(d->attn_cnt_, 0, static_cast<size_t>(c.n_heads) * sizeof(unsigned)), "hipMemset");
+    // Pinned host memory of the synchronous calls: state, logits, prompt tokens.
+    d->host_tokens_at_ = kHostLogitsAt + (static_cast<size_t>(c.vocab_size) * 4 + 255) / 256 * 256;
+    d->check(hipHostMalloc(&d->host_, d->host_tokens_at_ + static_cast<size_t>(c.max_seq_len) * 4, hipHostMallocDefault),
+             "hipHostMalloc");
     d->check(hipDeviceSynchronize(), "hipDeviceSynchronize");
     return d;
 }
@@ -1571,6 +1618,7 @@ Decoder::~Decoder() {
     for (hipEvent_t ev : inflight_)
         if (ev) (void)hipEventDestroy(ev);
     for (void* p : allocs_) (void)hipFree(p);
+    if (host_) (void)hipHostFree(host_);
     if (stream_) (void)hipStreamDestroy(stream_);
 }
 
@@ -2088,9 +2136,7 @@ void Decoder::prefill(const int* tokens, int n, int start, float* logits_host) {
     }
     ensure_io(static_cast<size_t>(n));
     ensure_prefill();
-    DecodeState st{};
-    check(hipMemcpyAsync(state_, &st, sizeof st, hipMemcpyHostToDevice, stream_), "hipMemcpyAsync");
-    check(hipMemcpyAsync(io_, tokens, static_cast<size_t>(n) * 4, hipMemcpyHostToDevice, stream_), "hipMemcpyAsync");
+    set_state(DecodeState{}, tokens, n);
     for (int c0 = 0; c0 < n; c0 += kPrefillRows) {
         const int rows = std::min(kPrefillRows, n - c0);
         enqueue_prefill(stream_, io_ + c0, rows, start + c0);
@@ -2101,14 +2147,30 @@ void Decoder::prefill(const int* tokens, int n, int start, float* logits_host) {
             linear_group(stream_, lm, lm_y, 1, H_ + static_cast<size_t>(rows - 1) * c.dim);
         }
     }
-    if (logits_host != nullptr) {
-        check(hipMemcpyAsync(logits_host, logits_, static_cast<size_t>(c.vocab_size) * 4, hipMemcpyDeviceToHost,
-                             stream_),
-              "hipMemcpyAsync");
-    }
-    check(hipMemcpyAsync(&st, state_, sizeof st, hipMemcpyDeviceToHost, stream_), "hipMemcpyAsync");
+    finish(logits_host);
+}
+
+// The state and n prompt tokens (into io_) ahead of a synchronous call's launches.
+void Decoder::set_state(const DecodeState& st, const int* tokens, int n) {
+    int32_t* const h = reinterpret_cast<int32_t*>(static_cast<char*>(host_) + host_tokens_at_);
+    if (n > 0) std::memcpy(h, tokens, static_cast<size_t>(n) * 4);
+    hipLaunchKernelGGL(set_state_kernel, dim3(std::max(1, std::min(64, (n + 1023) / 1024))), dim3(n > 0 ? 1024 : 64), 0,
+                       stream_, state_, st, h, n, io_);
+    check(hipGetLastError(), "set_state_kernel");
+}
+
+// Waits for the call's launches; the logits to `logits_host` (when not null).
+// Throws on an error the device flagged.
+void Decoder::finish(float* logits_host) {
+    char* const h = static_cast<char*>(host_);
+    const DecodeState* const st = reinterpret_cast<const DecodeState*>(h);
+    const int n = logits_host != nullptr ? cfg_.vocab_size : 0;
+    hipLaunchKernelGGL(publish_kernel, dim3(std::max(1, std::min(256, (n / 4 + 255) / 256))), dim3(256), 0, stream_, state_,
+                       logits_, n, reinterpret_cast<DecodeState*>(h), reinterpret_cast<float*>(h + kHostLogitsAt));
+    check(hipGetLastError(), "publish_kernel");
     check(hipStreamSynchronize(stream_), "hipStreamSynchronize");
-    if (st.error != 0) throw std::runtime_error("HIP decoder: device step reported error " + std::to_string(st.error));
+    if (n > 0) std::memcpy(logits_host, h + kHostLogitsAt, static_cast<size_t>(n) * 4);
+    if (st->error != 0) throw std::runtime_error("HIP decoder: device step reported error " + std::to_string(st->error));
 }
 
 void Decoder::ensure_io(size_t need) {
@@ -2133,13 +2195,10 @@ void Decoder::forward(int token, int pos, float* logits_host) {
     DecodeState st{};
     st.pos = pos;
     st.token = token;
-    check(hipMemcpyAsync(state_, &st, sizeof st, hipMemcpyHostToDevice, stream_), "hipMemcpyAsync");
+    if (logits_host == nullptr) check(hipErrorInvalidValue, "forward logits");
+    set_state(st, nullptr, 0);
     enqueue_step(stream_, false, false);
-    check(hipMemcpyAsync(logits_host, logits_, static_cast<size_t>(c.vocab_size) * 4, hipMemcpyDeviceToHost, stream_),
-          "hipMemcpyAsync");
-    check(hipMemcpyAsync(&st, state_, sizeof st, hipMemcpyDeviceToHost, stream_), "hipMemcpyAsync");
-    check(hipStreamSynchronize(stream_), "hipStreamSynchronize");
-    if (st.error != 0) throw std::runtime_error("HIP decoder: device step reported error " + std::to_string(st.error));
+    finish(logits_host);
 }
 
 void Decoder::generate(const int* prompt, int n_prompt, int n_new, int* out) {

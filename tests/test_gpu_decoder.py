@@ -296,3 +296,28 @@ def test_batched_prefill_longer_than_one_pass(hip, orc, ref, tmp_path):
     got = dec.generate(toks[:300], 8)
     assert got == ref.decoder(path).generate(toks[:300], 8)
     dec.close()
+
+
+@pytest.mark.parametrize("fmt", ["q4_0", "q8_0", "q4_1"])
+def test_prefill_equals_steps(hip, orc, tmp_path, fmt):
+    """The batched prefill against one step per token on the device (no reference
+    needed): a width whose prefill runs the large-tile GEMM with the norm and SwiGLU
+    kernels writing its split x, and steps at either side of every split of the
+    decode attention (one split per 128 positions, eight at most)."""
+    path = mf.write_model(orc, str(tmp_path / f"wide_{fmt}.gguf"), layers=1, dim=2048, hidden=2816, heads=16, kv_heads=8,
+                          vocab=500, ctx=1200, fmts=(fmt,), lm=fmt, seed=11, scale=0.02)
+    say(f"prefill against steps {fmt}")
+    dec = hip.Decoder(path)
+    tokens = np.random.default_rng(3).integers(0, 500, 1100)
+    at = {300, 127, 128, 129, 511, 512, 1024, 1025, 1099}
+    steps = {}
+    for pos, t in enumerate(tokens):
+        got = dec.forward(int(t), pos)
+        if pos in at:
+            steps[pos] = got
+    for pos in sorted(at):
+        worst = close(dec.prefill(tokens[:pos + 1]), steps[pos], f"{fmt} prefill of {pos + 1}")
+        say(f"  {pos + 1} tokens: {worst:.2e}")
+    with pytest.raises(hip.MlqError, match="position out of range"):
+        dec.forward(1, 1200)
+    dec.close()
