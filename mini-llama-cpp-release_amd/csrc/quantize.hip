@@ -7,15 +7,16 @@
 //   Q4_1              tests/test_cuda_quant.cpp:129-180 (the only Q4_1 quantizer
 //                     the reference has; its parity tests use it)
 // Every step is an IEEE f32 operation with one rounding (|v|, max, a / 127,
-// 1 / d, v * inv, v * inv + 8, (v - m) * inv) or integer work, so the device
-// result matches the host bit for bit: hipcc divides with correct rounding
-// (no fast-math), roundf rounds half away from zero like std::round, and no
-// expression here can be contracted into an fma.  The scale is encoded with the
+// 1 / d, v * inv, (v - m) * inv) or integer work, so the device result matches the
+// host bit for bit: hipcc divides with correct rounding (no fast-math), roundf
+// rounds half away from zero like std::round, and the kernel contracts nothing into
+// an fma by itself.  The one fma is Q4_0's v * inv + 8: a host that rounds the product
+// first differs from it in one byte of about 10^7 (ties made by that rounding).  The scale is encoded with the
 // reference's binary16 rule (round half up in magnitude at the first dropped
 // bit, overflow and NaN to Inf, src/quant.cpp:19-55), not the hardware cvt.
 //
-// One thread quantizes one block; a block's 32 floats are read as 8 float4 when
-// the row is 16-byte aligned and in range, element-wise otherwise.
+// Four lanes quantize one block; a lane reads two float4s where every row is 16-byte
+// aligned, element by element otherwise.
 
 #include "mlq_kernels.h"
 
@@ -61,111 +62,182 @@ template <> struct QB<1> { static constexpr int BB = 34; };
 template <> struct QB<2> { static constexpr int BB = 18; };
 template <> struct QB<3> { static constexpr int BB = 20; };
 
-template <int QT>
-__global__ __launch_bounds__(256) void quantize_kernel(const float* __restrict__ src, int rows,
-                                                       int row_len, uint8_t* __restrict__ dst) {
-    const int nb = (row_len + kQK - 1) / kQK;
-    const long long idx = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (idx >= static_cast<long long>(rows) * nb) return;
-    const int r = static_cast<int>(idx / nb);
-    const int b = static_cast<int>(idx % nb);
-    const float* p = src + static_cast<size_t>(r) * row_len + b * kQK;
-    const int len = min(kQK, row_len - b * kQK);
+// The other lane of the quad that differs in bit 0 (CTRL 0xB1) or bit 1 (0x4E).
+template <int CTRL>
+__device__ __forceinline__ float quad_peer(float v) {
+    return __builtin_bit_cast(
+        float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
+}
 
-    float v[kQK];
-    if (len == kQK && (reinterpret_cast<uintptr_t>(p) & 15u) == 0) {
+// Largest of a quad's values (none is NaN).
+__device__ __forceinline__ float quad_max(float v) {
+    float o = quad_peer<0xB1>(v);
+    v = (v < o) ? o : v;
+    o = quad_peer<0x4E>(v);
+    return (v < o) ? o : v;
+}
+
+// Smallest of a quad's values (none is NaN); of equal ones the lowest lane's, as a
+// scan in element order keeps it (it decides the sign of a zero).
+__device__ __forceinline__ float quad_first_min(float v, int l) {
+    float o = quad_peer<0xB1>(v);
+    v = (l & 1) ? ((v < o) ? v : o) : ((o < v) ? o : v);
+    o = quad_peer<0x4E>(v);
+    return (l & 2) ? ((v < o) ? v : o) : ((o < v) ? o : v);
+}
+
+constexpr int kQuantThreads = 256;
+constexpr int kQuantPasses = 2;
+constexpr int kQuantBlocks = kQuantThreads / 4 * kQuantPasses;  // blocks per workgroup
+
+// How a lane finds its elements: rows of whole blocks back to back (no division),
+// rows whose float4s are aligned and whole or absent, any rows.
+enum Rows { kWhole, kVector, kElement };
+
+// Bound: HBM (4 * row_len read, blocks written).  Four lanes take a block, lane l its
+// elements 4l..4l+3 and 16+4l..16+4l+3: both are one float4, a Q4 byte's two nibbles
+// are in one lane, and the block's extremes fold in two quad permutes.  The packed
+// blocks of the workgroup (kQuantBlocks of them, a multiple of 16 bytes) gather in LDS
+// and leave in 16-byte stores.  One thread per block
+// (128-byte strides between lanes, 16-bit stores) / this, us: 11008 x 4096 Q8_0 46.3 /
+// 41.2 (5.5 TB/s; a copy runs at 5.1), Q4_0 39.2 / 38.2, Q4_1 40.4 / 40.4; 10000 x 2500 Q8_0
+// 29.0 / 26.3; 16000 x 2051 Q4_0 69.7 / 58.7; 3000 x 896 Q4_0 5.2 / 4.1.
+template <int QT, Rows ROWS>
+__global__ __launch_bounds__(kQuantThreads) void quantize_kernel(const float* __restrict__ src,
+                                                                 long long total, int row_len,
+                                                                 uint8_t* __restrict__ dst,
+                                                                 bool wide) {
+#pragma clang fp contract(off)
+    constexpr int BB = QB<QT>::BB;
+    static_assert(kQuantBlocks * BB % 16 == 0, "a workgroup's blocks start 16-byte aligned");
+    __shared__ alignas(16) uint16_t packed[kQuantBlocks * BB / 2];
+    const int t = threadIdx.x;
+    const int l = t & 3;
+    const long long first = static_cast<long long>(blockIdx.x) * kQuantBlocks;
+    const int here = static_cast<int>(min(static_cast<long long>(kQuantBlocks), total - first));
+
+    float v[kQuantPasses][8];  // elements 4l.., then 16 + 4l..
+    int len[kQuantPasses];
 #pragma unroll
-        for (int i = 0; i < kQK / 4; ++i) {
-            const float4 f = reinterpret_cast<const float4*>(p)[i];
-            v[4 * i] = f.x;
-            v[4 * i + 1] = f.y;
-            v[4 * i + 2] = f.z;
-            v[4 * i + 3] = f.w;
+    for (int s = 0; s < kQuantPasses; ++s) {
+        // lanes past the last block repeat it (their result is not stored)
+        const int local = min(s * (kQuantThreads / 4) + (t >> 2), here - 1);
+        if (ROWS == kWhole) {
+            const float4* p = reinterpret_cast<const float4*>(src + (first + local) * kQK);
+            len[s] = kQK;
+            const float4 a = p[l];
+            const float4 b = p[4 + l];
+            v[s][0] = a.x, v[s][1] = a.y, v[s][2] = a.z, v[s][3] = a.w;
+            v[s][4] = b.x, v[s][5] = b.y, v[s][6] = b.z, v[s][7] = b.w;
+        } else {
+            const unsigned nb = (static_cast<unsigned>(row_len) + kQK - 1) / kQK;
+            const unsigned at = static_cast<unsigned>(first % nb) + local;
+            const float* p = src + static_cast<size_t>(first / nb + at / nb) * row_len + at % nb * kQK;
+            len[s] = min(kQK, row_len - static_cast<int>(at % nb) * kQK);
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int e = 16 * h + 4 * l;
+                if (ROWS == kVector) {
+                    float4 f = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                    if (e < len[s]) f = *reinterpret_cast<const float4*>(p + e);
+                    v[s][4 * h] = f.x, v[s][4 * h + 1] = f.y, v[s][4 * h + 2] = f.z, v[s][4 * h + 3] = f.w;
+                } else {
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) v[s][4 * h + c] = (e + c < len[s]) ? p[e + c] : 0.0f;
+                }
+            }
         }
-    } else {
-#pragma unroll
-        for (int i = 0; i < kQK; ++i) v[i] = (i < len) ? p[i] : 0.0f;
     }
 
-    uint8_t out[QB<QT>::BB];
 #pragma unroll
-    for (int i = 0; i < QB<QT>::BB; ++i) out[i] = 0;
-
-    if (QT == 1 || QT == 2) {
-        float amax = 0.0f;
+    for (int s = 0; s < kQuantPasses; ++s) {
+        uint16_t* out = packed + (s * (kQuantThreads / 4) + (t >> 2)) * (BB / 2);
+        if (QT == 1 || QT == 2) {
+            float amax = 0.0f;  // elements past the row are 0
 #pragma unroll
-        for (int i = 0; i < kQK; ++i) {
-            const float a = fabsf(v[i]);
-            if (i < len && a > amax) amax = a;
-        }
-        if (amax > 0.0f) {
-            const uint16_t dh = half_round_up(amax / (QT == 1 ? 127.0f : 7.0f));
+            for (int i = 0; i < 8; ++i) {
+                const float a = fabsf(v[s][i]);
+                amax = (a > amax) ? a : amax;
+            }
+            amax = quad_max(amax);
+            const bool some = amax > 0.0f;  // else the block is all zero bytes
+            const uint16_t dh = some ? half_round_up(amax / (QT == 1 ? 127.0f : 7.0f)) : 0;
             const float dq = half_value(dh);
             const float inv = (dq == 0.0f) ? 0.0f : 1.0f / dq;
-            out[0] = static_cast<uint8_t>(dh & 0xff);
-            out[1] = static_cast<uint8_t>(dh >> 8);
+            if (l == 0) out[0] = dh;
             if (QT == 1) {
+                int q[8];
 #pragma unroll
-                for (int i = 0; i < kQK; ++i) {
-                    int q = round_int(v[i] * inv);
-                    q = max(-127, min(127, q));
-                    out[2 + i] = static_cast<uint8_t>(static_cast<int8_t>(i < len ? q : 0));
+                for (int i = 0; i < 8; ++i) {
+                    q[i] = round_int(v[s][i] * inv);
+                    q[i] = some ? max(-127, min(127, q[i])) & 0xff : 0;
+                }
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    out[1 + 8 * h + 2 * l] = static_cast<uint16_t>(q[4 * h] | (q[4 * h + 1] << 8));
+                    out[2 + 8 * h + 2 * l] = static_cast<uint16_t>(q[4 * h + 2] | (q[4 * h + 3] << 8));
                 }
             } else {
+                int q[4];
 #pragma unroll
-                for (int j = 0; j < 16; ++j) {
-                    const float lo = (j < len) ? v[j] * inv : 0.0f;
-                    const float hi = (j + 16 < len) ? v[j + 16] * inv : 0.0f;
-                    const int qlo = max(0, min(15, round_int(lo + 8.0f)));
-                    const int qhi = max(0, min(15, round_int(hi + 8.0f)));
-                    out[2 + j] = static_cast<uint8_t>(qlo | (qhi << 4));
+                for (int j = 0; j < 4; ++j) {
+                    const int qlo = max(0, min(15, round_int(__builtin_fmaf(v[s][j], inv, 8.0f))));
+                    const int qhi = max(0, min(15, round_int(__builtin_fmaf(v[s][4 + j], inv, 8.0f))));
+                    q[j] = some ? qlo | (qhi << 4) : 0;
+                }
+                out[1 + 2 * l] = static_cast<uint16_t>(q[0] | (q[1] << 8));
+                out[2 + 2 * l] = static_cast<uint16_t>(q[2] | (q[3] << 8));
+            }
+        } else {
+            // std::min / std::max semantics in element order: the first of equal
+            // values stays, NaN never enters.
+            float lo[2] = {__builtin_inff(), __builtin_inff()};
+            float hi = -__builtin_inff();
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                if (16 * (i >> 2) + 4 * l + (i & 3) < len[s]) {
+                    lo[i >> 2] = (v[s][i] < lo[i >> 2]) ? v[s][i] : lo[i >> 2];
+                    hi = (hi < v[s][i]) ? v[s][i] : hi;
                 }
             }
-        }
-    } else {
-        float lo = __builtin_inff();
-        float hi = -__builtin_inff();
-#pragma unroll
-        for (int i = 0; i < kQK; ++i) {
-            if (i < len) {
-                // std::min / std::max semantics: keep the first operand unless
-                // the second compares strictly smaller / larger.
-                lo = (v[i] < lo) ? v[i] : lo;
-                hi = (hi < v[i]) ? v[i] : hi;
-            }
-        }
-        const float range = hi - lo;
-        uint16_t dh = 0;
-        uint16_t mh;
-        if (range > 0.0f) {
-            dh = half_round_up(range / 15.0f);
-            mh = half_round_up(lo);
+            lo[0] = quad_first_min(lo[0], l);
+            lo[1] = quad_first_min(lo[1], l);
+            const float mn = (lo[1] < lo[0]) ? lo[1] : lo[0];
+            const float range = quad_max(hi) - mn;
+            const bool some = range > 0.0f;
+            const uint16_t dh = some ? half_round_up(range / 15.0f) : 0;
+            const uint16_t mh = half_round_up((!some && mn == __builtin_inff()) ? 0.0f : mn);
             const float dq = half_value(dh);
             const float mq = half_value(mh);
             const float inv = (dq == 0.0f) ? 0.0f : 1.0f / dq;
+            if (l == 0) {
+                out[0] = dh;
+                out[1] = mh;
+            }
+            int q[4];
 #pragma unroll
-            for (int j = 0; j < 16; ++j) {
-                int q0 = (j < len) ? round_int((v[j] - mq) * inv) : 0;
-                int q1 = (j + 16 < len) ? round_int((v[j + 16] - mq) * inv) : 0;
+            for (int j = 0; j < 4; ++j) {
+                int q0 = (4 * l + j < len[s]) ? round_int((v[s][j] - mq) * inv) : 0;
+                int q1 = (16 + 4 * l + j < len[s]) ? round_int((v[s][4 + j] - mq) * inv) : 0;
                 q0 = max(0, min(15, q0));
                 q1 = max(0, min(15, q1));
-                out[4 + j] = static_cast<uint8_t>(q0 | (q1 << 4));
+                q[j] = some ? q0 | (q1 << 4) : 0;
             }
-        } else {
-            mh = half_round_up(lo == __builtin_inff() ? 0.0f : lo);
+            out[2 + 2 * l] = static_cast<uint16_t>(q[0] | (q[1] << 8));
+            out[3 + 2 * l] = static_cast<uint16_t>(q[2] | (q[3] << 8));
         }
-        out[0] = static_cast<uint8_t>(dh & 0xff);
-        out[1] = static_cast<uint8_t>(dh >> 8);
-        out[2] = static_cast<uint8_t>(mh & 0xff);
-        out[3] = static_cast<uint8_t>(mh >> 8);
     }
+    __syncthreads();
 
-    uint8_t* q = dst + static_cast<size_t>(idx) * QB<QT>::BB;
-    // Blocks are 2-byte aligned (Q4_1: 4-byte); store as 16-bit halves.
-    uint16_t* q16 = reinterpret_cast<uint16_t*>(q);
-#pragma unroll
-    for (int i = 0; i < QB<QT>::BB / 2; ++i) {
-        q16[i] = static_cast<uint16_t>(out[2 * i] | (out[2 * i + 1] << 8));
+    // `wide`: dst is 16-byte aligned; else, and for the last workgroup's remainder, 16-bit halves.
+    uint8_t* base = dst + static_cast<size_t>(first) * BB;
+    const int bytes = here * BB;
+    const int units = wide ? bytes / 16 : 0;
+    for (int u = t; u < units; u += kQuantThreads) {
+        reinterpret_cast<uint4*>(base)[u] = reinterpret_cast<const uint4*>(packed)[u];
+    }
+    for (int h = units * 8 + t; h < bytes / 2; h += kQuantThreads) {
+        reinterpret_cast<uint16_t*>(base)[h] = packed[h];
     }
 }
 
@@ -196,10 +268,19 @@ __global__ __launch_bounds__(256) void fill_normal_kernel(float* __restrict__ ds
 
 template <int QT>
 hipError_t launch_q(const float* src, int rows, int row_len, void* dst, hipStream_t stream) {
-    const long long n = static_cast<long long>(rows) * ((row_len + kQK - 1) / kQK);
-    const long long grid = (n + 255) / 256;
-    hipLaunchKernelGGL((quantize_kernel<QT>), dim3(static_cast<unsigned>(grid)), dim3(256), 0,
-                       stream, src, rows, row_len, static_cast<uint8_t*>(dst));
+    const long long n = static_cast<long long>(rows) * ((static_cast<long long>(row_len) + kQK - 1) / kQK);
+    const dim3 grid(static_cast<unsigned>((n + kQuantBlocks - 1) / kQuantBlocks));
+    uint8_t* out = static_cast<uint8_t*>(dst);
+    const bool wide = (reinterpret_cast<uintptr_t>(dst) & 15u) == 0;
+    // A float4 needs its 16-byte alignment: the source's and, in every row, the length's.
+    const bool vec = (reinterpret_cast<uintptr_t>(src) & 15u) == 0 && row_len % 4 == 0;
+    if (vec && row_len % kQK == 0) {
+        quantize_kernel<QT, kWhole><<<grid, kQuantThreads, 0, stream>>>(src, n, row_len, out, wide);
+    } else if (vec) {
+        quantize_kernel<QT, kVector><<<grid, kQuantThreads, 0, stream>>>(src, n, row_len, out, wide);
+    } else {
+        quantize_kernel<QT, kElement><<<grid, kQuantThreads, 0, stream>>>(src, n, row_len, out, wide);
+    }
     return hipGetLastError();
 }
 

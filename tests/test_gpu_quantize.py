@@ -59,6 +59,37 @@ def test_device_quantizer_random_and_special(hip, orc, fmt):
         assert np.array_equal(device_quantize(hip, qt, w), orc.quantize(qt, w, threads=4)), w.shape
 
 
+@pytest.mark.parametrize("fmt", list(FMTS))
+@pytest.mark.parametrize("rows,k", [(1, 32), (1, 127 * 32), (1, 128 * 32), (129, 32), (3, 43 * 32),  # whole blocks
+                                    (1, 4), (5, 36), (130, 44), (7, 4092),                           # float4s, a tail
+                                    (1, 1), (131, 33), (9, 31), (2, 4097)])                          # elements
+@pytest.mark.parametrize("off", [0, 2])
+def test_device_quantizer_edges(hip, orc, fmt, rows, k, off):
+    """Workgroups of 128 blocks, their remainders, and each way rows are read; blocks
+    stored in 16-byte units or (at an offset) in halves, nothing past them; the first
+    of equal minima stays (its zero's sign is in a Q4_1 block)."""
+    qt = FMTS[fmt]
+    rng = np.random.default_rng(rows * 5000 + k)
+    w = rng.standard_normal((rows, k), dtype=np.float32)
+    zeros = rng.random((rows, k)) < 0.4
+    w[rows // 2:] = np.abs(w[rows // 2:])
+    w[zeros] = np.where(rng.random(int(zeros.sum())) < 0.5, np.float32(0.0), np.float32(-0.0))
+    nb = (k + 31) // 32
+    size = rows * nb * oracle.BLOCK_BYTES[qt]
+    src = hip.DeviceBuffer.from_array(w)
+    dst = hip.DeviceBuffer(size + 64)
+    dst.fill(0xAB)
+
+    class At:
+        ptr, nbytes = dst.ptr + off, size
+    print(f"quantize edges {fmt} {rows} x {k} at {off}", flush=True)
+    hip.quantize_device(qt, src, rows, k, At)
+    hip.synchronize(hip.stream(0))
+    got = dst.download(np.uint8)
+    assert np.array_equal(got[off:off + size].reshape(rows * nb, -1), orc.quantize(qt, w, threads=4))
+    assert (got[:off] == 0xAB).all() and (got[off + size:] == 0xAB).all()
+
+
 def test_fill_normal_moments(hip):
     n = 1 << 22
     buf = hip.DeviceBuffer(4 * n)
