@@ -7,13 +7,14 @@
 //   Q4_1              tests/test_cuda_quant.cpp:129-180 (the only Q4_1 quantizer
 //                     the reference has; its parity tests use it)
 // Every step is an IEEE f32 operation with one rounding (|v|, max, a / 127,
-// 1 / d, v * inv, (v - m) * inv) or integer work, so the device result matches the
-// host bit for bit: hipcc divides with correct rounding (no fast-math), roundf
-// rounds half away from zero like std::round, and the kernel contracts nothing into
-// an fma by itself.  The one fma is Q4_0's v * inv + 8: a host that rounds the product
-// first differs from it in one byte of about 10^7 (ties made by that rounding).  The scale is encoded with the
-// reference's binary16 rule (round half up in magnitude at the first dropped
-// bit, overflow and NaN to Inf, src/quant.cpp:19-55), not the hardware cvt.
+// 1 / d, v * inv, its sum with 8, (v - m) * inv) or integer work, so the device result
+// matches the host bit for bit: hipcc divides with correct rounding (no fast-math),
+// roundf rounds half away from zero like std::round, and nothing is contracted into an
+// fma (contract(off) below): Q4_0's v * inv + 8 as one would move codes whose product
+// rounds onto a tie, 1e-7 of them for f32 normal weights, 1e-4 for bf16 ones, 8e-4 for
+// integers up to 100.  The scale is encoded with the reference's binary16 rule (round half
+// up in magnitude at the first dropped bit, overflow and NaN to Inf,
+// src/quant.cpp:19-55), not the hardware cvt.
 //
 // Four lanes quantize one block; a lane reads two float4s where every row is 16-byte
 // aligned, element by element otherwise.
@@ -181,8 +182,8 @@ __global__ __launch_bounds__(kQuantThreads) void quantize_kernel(const float* __
                 int q[4];
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    const int qlo = max(0, min(15, round_int(__builtin_fmaf(v[s][j], inv, 8.0f))));
-                    const int qhi = max(0, min(15, round_int(__builtin_fmaf(v[s][4 + j], inv, 8.0f))));
+                    const int qlo = max(0, min(15, round_int(v[s][j] * inv + 8.0f)));
+                    const int qhi = max(0, min(15, round_int(v[s][4 + j] * inv + 8.0f)));
                     q[j] = some ? qlo | (qhi << 4) : 0;
                 }
                 out[1 + 2 * l] = static_cast<uint16_t>(q[0] | (q[1] << 8));

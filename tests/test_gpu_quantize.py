@@ -90,6 +90,31 @@ def test_device_quantizer_edges(hip, orc, fmt, rows, k, off):
     assert (got[:off] == 0xAB).all() and (got[off + size:] == 0xAB).all()
 
 
+def coarse_weights(kind, rows, k):
+    """Weights as checkpoints hold them, on grids whose products land on ties."""
+    rng = np.random.default_rng(77)
+    if kind == "integers":
+        return rng.integers(-100, 101, (rows, k)).astype(np.float32)
+    w = rng.standard_normal((rows, k), dtype=np.float32) * np.float32(0.02)
+    if kind == "fp16":
+        return w.astype(np.float16).astype(np.float32)
+    return (w.view(np.uint32) & np.uint32(0xffff0000)).view(np.float32)  # bf16
+
+
+@pytest.mark.parametrize("fmt", list(FMTS))
+@pytest.mark.parametrize("kind", ["integers", "fp16", "bf16"])
+def test_device_quantizer_coarse_values(hip, orc, fmt, kind):
+    """Every operation rounded by itself, as the host rounds it.  A product fused with
+    the sum after it moves codes whose rounded product is a tie: Q4_0 of -65 beside
+    a block maximum of 70 is 1.5 rounded, 1.49999994 fused."""
+    qt = FMTS[fmt]
+    w = coarse_weights(kind, 512, 4096)
+    w[0, :2] = (70, -65)
+    w[0, 2:32] = 0
+    print(f"quantize {fmt} {kind}", flush=True)
+    assert np.array_equal(device_quantize(hip, qt, w), orc.quantize(qt, w, threads=4))
+
+
 def test_fill_normal_moments(hip):
     n = 1 << 22
     buf = hip.DeviceBuffer(4 * n)
