@@ -647,7 +647,7 @@ __global__ __launch_bounds__(256) void add_rmsnorm_split_rows_kernel(float* __re
         }
     }
     __syncthreads();  // part is reused by the split's maximum
-    xsplit_emit_row<QT, C, true>(row, nb, v, xs, bsum, scale, part);
+    xsplit_emit_row<QT, C>(row, nb, v, xs, bsum, scale, part);
 }
 
 // swiglu_kernel's step for a GEMM input: the split of silu(g) * u per row.
@@ -681,7 +681,7 @@ __global__ __launch_bounds__(256) void swiglu_split_rows_kernel(const float* __r
             v[c][i] = in ? gv * sig * uv[c][i] : 0.0f;
         }
     }
-    xsplit_emit_row<QT, C, true>(row, nb, v, xs, bsum, scale, red);
+    xsplit_emit_row<QT, C>(row, nb, v, xs, bsum, scale, red);
 }
 
 // rope_kv_kernel for every row (position start + r): workgroups (0 .. R-1,

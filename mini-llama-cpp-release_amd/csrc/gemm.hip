@@ -73,7 +73,7 @@ __device__ __forceinline__ int slot_k(int g, int j) {
 // row, then the scaled split), so rows up to 16 384 elements are read once; longer
 // rows re-read the rest (L2 hits).  The split itself is xsplit_device.h's, which
 // kernels producing a GEMM input also use.
-template <int QT, bool PACK, int C>
+template <int QT, int C>
 __global__ __launch_bounds__(256) void xsplit_kernel(const float* __restrict__ x, int N, int K, int nb,
                                                      _Float16* __restrict__ xs, float* __restrict__ bsum,
                                                      float* __restrict__ scale) {
@@ -119,7 +119,7 @@ __global__ __launch_bounds__(256) void xsplit_kernel(const float* __restrict__ x
         for (int c = 0; c < C; ++c) load8(threadIdx.x + 256 * c, cache[c]);
     }
     if (items <= 256 * C) {
-        xsplit_emit_row<QT, C, PACK>(n, nb, cache, xs, bsum, scale, red);
+        xsplit_emit_row<QT, C>(n, nb, cache, xs, bsum, scale, red);
         return;
     }
     float mx = 0.0f;
@@ -139,29 +139,29 @@ __global__ __launch_bounds__(256) void xsplit_kernel(const float* __restrict__ x
     if (threadIdx.x == 0) scale[n] = sc;
     const int iters = (items + 255) / 256;  // uniform across the workgroup
 #pragma unroll
-    for (int c = 0; c < C; ++c) xsplit_emit_item<QT, PACK>(n, nb, threadIdx.x + 256 * c, cache[c], inv, xs, bsum);
+    for (int c = 0; c < C; ++c) xsplit_emit_item<QT>(n, nb, threadIdx.x + 256 * c, cache[c], inv, xs, bsum);
     for (int it = C; it < iters; ++it) {
         float v[8];
         const int i = threadIdx.x + 256 * it;
         load8(i, v);
-        xsplit_emit_item<QT, PACK>(n, nb, i, v, inv, xs, bsum);
+        xsplit_emit_item<QT>(n, nb, i, v, inv, xs, bsum);
     }
 }
 
-template <int QT, bool PACK>
+template <int QT>
 void launch_xsplit(const float* x, int rows, int K, int nb, int npad, _Float16* xs, float* bsum, float* scale,
                    hipStream_t stream) {
     auto go = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3(npad), dim3(256), 0, stream, x, rows, K, nb, xs, bsum, scale);
     };
     if (nb <= 64) {
-        go(xsplit_kernel<QT, PACK, 1>);
+        go(xsplit_kernel<QT, 1>);
     } else if (nb <= 128) {
-        go(xsplit_kernel<QT, PACK, 2>);
+        go(xsplit_kernel<QT, 2>);
     } else if (nb <= 256) {
-        go(xsplit_kernel<QT, PACK, 4>);
+        go(xsplit_kernel<QT, 4>);
     } else {
-        go(xsplit_kernel<QT, PACK, kXsCache>);
+        go(xsplit_kernel<QT, kXsCache>);
     }
 }
 
@@ -1006,7 +1006,7 @@ hipError_t launch_t(const LinearShape& s, const GemmCfg& c, const WsLayout& l, c
     float* scale = reinterpret_cast<float*>(ws + l.scale);
     float* part = c.splits > 1 ? reinterpret_cast<float*>(ws + l.part) : nullptr;
     unsigned* count = reinterpret_cast<unsigned*>(ws + l.count);
-    launch_xsplit<QT, false>(x, s.rows, s.K, s.nb, c.npad, xs, bsum, scale, stream);
+    launch_xsplit<QT>(x, s.rows, s.K, s.nb, c.npad, xs, bsum, scale, stream);
     dim3 grid((s.M + 64 * RT - 1) / (64 * RT), c.npad / (16 * TT), c.splits);
     constexpr int lds = StreamLds<TT>::bytes;
     hipLaunchKernelGGL((gemm_stream_kernel<QT, RT, TT, (RT == 1 ? 4 : 2)>), grid, dim3(kGemmThreads), lds, stream,
@@ -1283,7 +1283,7 @@ hipError_t launch_tile(const LinearShape& s, const GemmPlan& c, const float* x, 
     a.tile1 = grp.n >= 2 ? grp.M[0] / kTileM : c.row_tiles;
     a.tile2 = grp.n >= 3 ? a.tile1 + grp.M[1] / kTileM : c.row_tiles;
     a.xs = reinterpret_cast<const _Float16*>(ws + c.ws.xs);
-    a.bsum = reinterpret_cast<const uint32_t*>(ws + c.ws.bsum);
+    a.bsum = reinterpret_cast<const float*>(ws + c.ws.bsum);
     a.xscale = reinterpret_cast<const float*>(ws + c.ws.scale);
     a.part = reinterpret_cast<float*>(ws + c.ws.part);
     a.part_bytes = static_cast<uint32_t>(c.ws.part_bytes);
@@ -1293,7 +1293,7 @@ hipError_t launch_tile(const LinearShape& s, const GemmPlan& c, const float* x, 
     a.xcd_br = a.xcd_row_outer = 0;
     if (c.splits == 1) xcd_blocks(s, c.row_tiles, c.tok_tiles, kTileM, kTileN, &a.xcd_br, &a.xcd_row_outer);
     if (!presplit) {
-        launch_xsplit<QT, true>(x, s.rows, s.K, s.nb, c.npad, reinterpret_cast<_Float16*>(ws + c.ws.xs),
+        launch_xsplit<QT>(x, s.rows, s.K, s.nb, c.npad, reinterpret_cast<_Float16*>(ws + c.ws.xs),
                                 reinterpret_cast<float*>(ws + c.ws.bsum), reinterpret_cast<float*>(ws + c.ws.scale), stream);
     }
     hipLaunchKernelGGL(kern, dim3(c.row_tiles * c.tok_tiles * c.splits), dim3(T::threads), T::lds, stream, a);

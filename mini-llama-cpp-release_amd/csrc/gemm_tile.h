@@ -23,6 +23,11 @@
 // together they held every wave at the start of the step: 47 -> 41.5 us).  The next
 // block is read from LDS and decoded while the current one is on the matrix cores;
 // a tile's scale fmas run under the next tile's MFMAs.  One barrier per step.
+// Q4_1's offset term m * sum(x') is an f32 product on the matrix cores, one
+// v_mfma_f32_32x32x1_2b_f32 (K = 1, both token tiles) per row tile and block: the
+// sums stay f32 and an infinite m meets no padding.  64 cycles for two tiles, what
+// two fp16 instructions on the sums' halves took (call, us, halves / f32: 4096 x 4096
+// at 512 tokens 52.3 / 52.0, q/k/v at 2048 546 / 545, gate/up at 300 172.4 / 172.9).
 // Measured (kernel alone, us; the 128 x 32-token kernel it replaced in brackets):
 // 4096 x 4096, 512 tokens Q4_0 41.5 (58), Q8_0 48 (66), Q4_1 47 (75);
 // 11008 x 4096 Q4_0 128 (165).
@@ -41,6 +46,7 @@ typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x32 __attribute__((ext_vector_type(32)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kTileBlocks = 4;  // blocks of K per step
@@ -85,7 +91,7 @@ struct TileArgs {
     int M[3];
     int tile1, tile2;       // first row tile of weights 1 and 2 (row_tiles when absent)
     const _Float16* xs;     // split x [npad][nb][64]
-    const uint32_t* bsum;   // Q4_1: block sums [npad][nb], packed hi and lo halves of sum / 32
+    const float* bsum;      // Q4_1: block sums [npad][nb]
     const float* xscale;    // [npad]
     float* part;
     uint32_t part_bytes;
@@ -233,11 +239,11 @@ __global__ __launch_bounds__(64 * NWM * NWN * KS, (NWM * NWN * KS + 3) / 4) void
     uint32_t mask = 0x000F000Fu, mask4 = 0x00F000F0u, magic = 0x64006400u;
     asm volatile("" : "+v"(mask), "+v"(mask4), "+v"(magic));
 
-    f32x16 acc[WM][WN];
+    // A row tile's sums: token tile t in elements 16 t .. 16 t + 15.
+    static_assert(WN == 2, "the block sums' product takes both token tiles");
+    f32x32 acc[WM];
 #pragma unroll
-    for (int r = 0; r < WM; ++r)
-#pragma unroll
-        for (int t = 0; t < WN; ++t) acc[r][t] = f32x16{};
+    for (int r = 0; r < WM; ++r) acc[r] = f32x32{};
     const f32x16 zero{};
 
     // A step's operands of this wave: its blocks' decoded weights, scales and x.
@@ -245,10 +251,9 @@ __global__ __launch_bounds__(64 * NWM * NWN * KS, (NWM * NWN * KS + 3) / 4) void
         f16x8 w[WM][2];
         _Float16 d[WM];
         f16x8 hi[WN][2], lo[WN][2];
-        uint32_t m[QT == 3 ? WM : 1], s[QT == 3 ? WN : 1];  // Q4_1: m twice; the block sum's halves
+        uint32_t dm[QT == 3 ? WM : 1];  // Q4_1: d and m as stored
+        float s;                        // Q4_1: block sum of token l32 of token tile h
     };
-    // Q4_1 accumulates y / 32: its block sums' halves stay within fp16.
-    constexpr float kUnit = QT == 3 ? 0.03125f : 1.0f;
     const int sw = x_swizzle(l32);
     uint32_t xu[2][2];
 #pragma unroll
@@ -264,17 +269,14 @@ __global__ __launch_bounds__(64 * NWM * NWN * KS, (NWM * NWN * KS + 3) / 4) void
             f.hi[t][s] = *reinterpret_cast<const f16x8*>(xt + xu[s][0]);
             f.lo[t][s] = *reinterpret_cast<const f16x8*>(xt + xu[s][1]);
         }
-        if (QT == 3) {
-            const uint32_t v = *reinterpret_cast<const uint32_t*>(smem + st + T::x_bytes +
-                                                                  ((wn * WN + t) * 32 + l32) * 16 + j * 4);
-            f.s[t] = h == 0 ? v : 0u;
-        }
+        if (QT == 3 && t == 0)
+            f.s = *reinterpret_cast<const float*>(smem + st + T::x_bytes + (wn * WN * 32 + lane) * 16 + j * 4);
     };
     auto read_w = [&](uint32_t st, int j, int r, uint32_t (&raw)[ND], Frag& f) {
         const char* row = smem + st + wrow0 + r * (32 * T::WROW);
         const uint32_t* pw = reinterpret_cast<const uint32_t*>(row);
         if (QT == 3) {
-            f.m[r] = pw[5 * j];
+            f.dm[r] = pw[5 * j];
 #pragma unroll
             for (int i = 0; i < ND; ++i) raw[i] = pw[5 * j + 1 + 2 * h + i];
             return;
@@ -291,8 +293,7 @@ __global__ __launch_bounds__(64 * NWM * NWN * KS, (NWM * NWN * KS + 3) / 4) void
 #pragma unroll
         for (int i = 0; i + 1 < ND; ++i) q[i] = __builtin_amdgcn_alignbit(raw[i + 1], raw[i], sh);
         if (QT == 3) {
-            f.d[r] = __builtin_bit_cast(h2_t, f.m[r]).x;
-            f.m[r] = h == 0 ? __builtin_amdgcn_perm(f.m[r], f.m[r], 0x07060706u) : 0u;
+            f.d[r] = __builtin_bit_cast(h2_t, f.dm[r]).x;
             f.w[r][0] = nibbles_f16<0>(raw[0], mask, mask4, magic);
             f.w[r][1] = nibbles_f16<0>(raw[1], mask, mask4, magic);
         } else if (QT == 1) {
@@ -332,17 +333,17 @@ __global__ __launch_bounds__(64 * NWM * NWN * KS, (NWM * NWN * KS + 3) / 4) void
             issue(c + ST, st_c, k, NT);
             if (r == WM - 1) read_x(st_n, j, t, nxt);
             const int kp = (k + NT - 1) % NT;  // the tile before
-            f32x16& ap = acc[kp % WM][kp / WM];
+            f32x32& ap = acc[kp % WM];
 #pragma unroll
-            for (int i = 0; i < 16; ++i) ap[i] = __builtin_fmaf(dprev, C[(k + 1) & 1][i], ap[i]);
-            if (QT == 3) {
-                // + m * sum(x'): the sum's halves against m in two of the k slots.
-                const u32x4 sa{cur.s[t], 0u, 0u, 0u}, mb{cur.m[r], 0u, 0u, 0u};
-                acc[r][t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, sa), __builtin_bit_cast(f16x8, mb),
-                                                                   acc[r][t], 0, 0, 0);
+            for (int i = 0; i < 16; ++i) ap[kp / WM * 16 + i] = __builtin_fmaf(dprev, C[(k + 1) & 1][i], ap[kp / WM * 16 + i]);
+            if (QT == 3 && k >= 1 && k <= WM) {
+                // + m * sum(x'), one k: both token tiles of a row tile (lanes 0-31 and
+                // 32-63 of the sums), between that row tile's two rounds of scale fmas.
+                const float m = static_cast<float>(__builtin_bit_cast(h2_t, cur.dm[kp % WM]).y);
+                ap = __builtin_amdgcn_mfma_f32_32x32x1f32(cur.s, m, ap, 0, 0, 0);
             }
             C[k & 1] = v;
-            dprev = static_cast<float>(cur.d[r]) * kUnit;
+            dprev = static_cast<float>(cur.d[r]);
             if (NT - k <= WM) decode_w(j, k + WM - NT, raw[k + WM - NT], nxt);
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -372,9 +373,9 @@ __global__ __launch_bounds__(64 * NWM * NWN * KS, (NWM * NWN * KS + 3) / 4) void
             step(c, A, B);
             step(c + 1, B, A);
         }
-        f32x16& ap = acc[WM - 1][WN - 1];
+        f32x32& ap = acc[WM - 1];
 #pragma unroll
-        for (int i = 0; i < 16; ++i) ap[i] = __builtin_fmaf(dprev, C[(WM * WN - 1) & 1][i], ap[i]);
+        for (int i = 0; i < 16; ++i) ap[16 + i] = __builtin_fmaf(dprev, C[(WM * WN - 1) & 1][i], ap[16 + i]);
         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // no copy may land in the reduction below
     }
 
@@ -383,8 +384,9 @@ __global__ __launch_bounds__(64 * NWM * NWN * KS, (NWM * NWN * KS + 3) / 4) void
     constexpr int GR = T::G / T::RR, GKR = T::GK / T::RR;
     auto group_of = [&](int q) { return (q / GKR) * GR + ks * GKR + q % GKR; };
     auto acc4 = [&](int g) {
-        const f32x16& v = acc[g / 4 / WN][g / 4 % WN];
-        return f32x4{v[4 * (g % 4)], v[4 * (g % 4) + 1], v[4 * (g % 4) + 2], v[4 * (g % 4) + 3]};
+        const f32x32& v = acc[g / 4 / WN];
+        const int i = 16 * (g / 4 % WN) + 4 * (g % 4);
+        return f32x4{v[i], v[i + 1], v[i + 2], v[i + 3]};
     };
     f32x4 own[T::GK];
     if (KS > 1) {
@@ -461,7 +463,7 @@ __global__ __launch_bounds__(64 * NWM * NWN * KS, (NWM * NWN * KS + 3) / 4) void
         const int n0 = n_base + (wn * WN + ttile) * 32 + 8 * (g % 4) + 4 * h;
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-            if (n0 + i < a.N && row < M) yg[static_cast<size_t>(n0 + i) * M + row] = own[q][i] * (1.0f / kUnit) * a.xscale[n0 + i];
+            if (n0 + i < a.N && row < M) yg[static_cast<size_t>(n0 + i) * M + row] = own[q][i] * a.xscale[n0 + i];
     }
 }
 

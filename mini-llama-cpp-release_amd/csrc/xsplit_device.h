@@ -37,8 +37,6 @@ __device__ __forceinline__ constexpr int xs_second() {
 }
 
 typedef _Float16 xs_h8 __attribute__((ext_vector_type(8)));
-typedef _Float16 xs_h2 __attribute__((ext_vector_type(2)));
-typedef _Float16 xs_h4 __attribute__((ext_vector_type(4)));
 
 // max |x| over the workgroup (every thread gets it); `red` is 4 floats of LDS.
 __device__ __forceinline__ float xsplit_row_max(float mx, float* red) {
@@ -65,9 +63,7 @@ __device__ __forceinline__ void xsplit_scale(float mx, float& inv, float& sc) {
 // Scales, splits and stores item i of token row n (v: its two runs).  Called by
 // every lane (a block's four items are on adjacent lanes); items past the row
 // store nothing.
-// PACK: the block sum as the two fp16 halves of sum / 32 (|sum| <= 2^19), which
-// the large-tile GEMM multiplies on the matrix cores.
-template <int QT, bool PACK>
+template <int QT>
 __device__ __forceinline__ void xsplit_emit_item(int n, int nb, int i, float (&v)[8], float inv,
                                                  _Float16* __restrict__ xs, float* __restrict__ bsum) {
 #pragma unroll
@@ -79,15 +75,7 @@ __device__ __forceinline__ void xsplit_emit_item(int n, int nb, int i, float (&v
     if (i >= 4 * nb) return;
     const int g = i & 3;
     const size_t b = static_cast<size_t>(n) * nb + (i >> 2);
-    if (g == 0) {
-        if (PACK) {
-            const _Float16 sh = static_cast<_Float16>(sum * 0.03125f);
-            const _Float16 sl = static_cast<_Float16>(sum * 0.03125f - static_cast<float>(sh));
-            reinterpret_cast<xs_h2*>(bsum)[b] = xs_h2{sh, sl};
-        } else {
-            bsum[b] = sum;
-        }
-    }
+    if (g == 0) bsum[b] = sum;
     xs_h8 hi, lo;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
@@ -105,7 +93,7 @@ __device__ __forceinline__ void xsplit_emit_item(int n, int nb, int i, float (&v
 // The whole split of token row n from the values the workgroup holds (thread
 // t: items t + 256 c in v[c], zeros past the row; 4 nb <= 256 C): the row's
 // maximum, its scale (stored by thread 0) and every item.
-template <int QT, int C, bool PACK>
+template <int QT, int C>
 __device__ __forceinline__ void xsplit_emit_row(int n, int nb, float (&v)[C][8], _Float16* __restrict__ xs,
                                                 float* __restrict__ bsum, float* __restrict__ scale, float* red) {
     float mx = 0.0f;
@@ -120,7 +108,7 @@ __device__ __forceinline__ void xsplit_emit_row(int n, int nb, float (&v)[C][8],
     const int iters = (4 * nb + 255) / 256;  // uniform across the workgroup
 #pragma unroll
     for (int c = 0; c < C; ++c)
-        if (c < iters) xsplit_emit_item<QT, PACK>(n, nb, static_cast<int>(threadIdx.x) + 256 * c, v[c], inv, xs, bsum);
+        if (c < iters) xsplit_emit_item<QT>(n, nb, static_cast<int>(threadIdx.x) + 256 * c, v[c], inv, xs, bsum);
 }
 
 // One float4 of `p` into v[k .. k + 3].

@@ -109,6 +109,54 @@ def test_gemm_large_tile_needs_dword_weights(hip, orc):
         buf.free()
 
 
+# The kernel of each shape: (out, in, rows, name part).
+KERNELS = [(4097, 1664, 333, "_tile_"), (300, 896, 40, "_chunk_"), (300, 4160, 40, "_q4_1_bm")]
+
+
+@pytest.mark.parametrize("m,k,n,part", KERNELS)
+def test_gemm_q4_1_offsets_in_f32(hip, m, k, n, part):
+    """Q4_1's offset term carries the block sums of x in 32 bits: with scales of 0 and
+    one offset of 1 per row, an output is one block's sum, here one 24-bit value."""
+    qt, nb = FMTS["q4_1"], k // 32
+    assert part in hip.kernel_name(qt, n, m, k)
+    rng = np.random.default_rng(8)
+    x = np.zeros((n, nb, 32), np.float32)
+    sums = (1 + rng.integers(0, 1 << 22, (n, nb)) * 2.0 ** -22 + 2.0 ** -23).astype(np.float32)
+    x[:, :, 5] = sums
+    at = np.arange(m) % nb
+    blocks = rng.integers(0, 256, (m, nb, 20), dtype=np.uint8)
+    head = blocks[:, :, :4].copy().view(np.float16)
+    head[:] = 0
+    head[np.arange(m), at, 1] = 1
+    blocks[:, :, :4] = head.view(np.uint8)
+    print(f"gemm q4_1 offsets M={m} K={k} N={n}", flush=True)
+    wt = hip.Weight.upload(qt, blocks.reshape(m * nb, 20), m, k)
+    got = wt.linear_host(x.reshape(n, k))
+    wt.free()
+    assert np.array_equal(got, sums[:, at])
+
+
+@pytest.mark.parametrize("m,k,n,part", KERNELS)
+def test_gemm_q4_1_infinite_offset(hip, orc, m, k, n, part):
+    """An infinite offset gives infinite outputs, not NaN."""
+    qt, nb = FMTS["q4_1"], k // 32
+    rng = np.random.default_rng(9)
+    x = np.abs(rng.standard_normal((n, k), dtype=np.float32)) + np.float32(0.01)
+    w = rng.standard_normal((m, k), dtype=np.float32) * np.float32(0.02)
+    blocks = orc.quantize(qt, w, threads=THREADS).reshape(m, nb, 20)
+    for row, b, v in ((0, 0, np.inf), (7, nb - 1, -np.inf), (m - 1, nb // 2, np.inf)):
+        blocks[row, b, 2:4] = np.array([v], np.float16).view(np.uint8)
+    blocks = blocks.reshape(m * nb, 20)
+    want = orc.linear(qt, x, blocks, m, threads=THREADS)
+    assert np.isinf(want[:, [0, 7, m - 1]]).all()
+    print(f"gemm q4_1 infinite offset M={m} K={k} N={n}", flush=True)
+    wt = hip.Weight.upload(qt, blocks, m, k)
+    got = wt.linear_host(x)
+    wt.free()
+    assert np.array_equal(got[:, [0, 7, m - 1]], want[:, [0, 7, m - 1]])
+    assert np.isfinite(np.delete(got, [0, 7, m - 1], axis=1)).all()
+
+
 def test_gemm_wide_dynamic_range(hip, orc):
     """Per-token power-of-two scaling keeps the hi/lo split exact across token
     magnitudes from 1e-6 to 1e4 (and an all-zero token)."""
