@@ -1935,8 +1935,8 @@ bool Decoder::prefill_batched() const {
 // every layer for all rows at once; X_ row n-1 ends as the last token's
 // residual stream (its final norm and lm_head are the caller's).
 // Where the GEMM of `ng` weights over `rows` rows reads a split x that the
-// kernel producing its input can write itself (same qtype and K for all, a
-// chunk GEMM that splits x, K <= 16 384); false: the usual plain-x path.
+// kernel producing its input can write itself (same qtype and K for all, the
+// large-tile GEMM, K <= 16 384); false: the usual plain-x path.
 bool Decoder::split_target(int ng, const Linear* const* w, int rows, SplitTarget& t) const {
     for (int g = 0; g < ng; ++g) {
         if (w[g]->qtype == 0 || w[g]->qtype != w[0]->qtype || w[g]->K != w[0]->K) return false;
@@ -1948,7 +1948,7 @@ bool Decoder::split_target(int ng, const Linear* const* w, int rows, SplitTarget
     t.ng = ng;
     t.shape = LinearShape{w[0]->qtype, 0, K, K / 32, rows};
     for (int g = 0; g < ng; ++g) t.shape.M += t.M[g];
-    t.sx = gemm_split_x(t.shape, ng, t.M);
+    t.sx = gemm_split_x(t.shape, ng, t.w, t.M);
     return t.sx.ok;
 }
 

@@ -524,7 +524,7 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_stream_kernel(
 // its partial tile with write-through stores and counts in; the workgroup
 // that completes the count adds the partials in split order (deterministic)
 // and writes y.  Needs nb % 4 == 0 (8-byte aligned
-// chunk rows), K == 32 nb and a 16-byte aligned x.
+// chunk rows) and K == 32 nb.
 constexpr int kChunkBlocks = 4;
 
 template <int QT> struct ChunkFmt;
@@ -661,7 +661,8 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_chunk_kernel(const ChunkArg
         }
     };
     auto load_x = [&](int c) {
-        const u32x4* src = reinterpret_cast<const u32x4*>(xrow + static_cast<size_t>(c) * 128);
+        typedef u32x4 x4_t __attribute__((aligned(4)));  // x starts on any float
+        const x4_t* src = reinterpret_cast<const x4_t*>(xrow + static_cast<size_t>(c) * 128);
 #pragma unroll
         for (int i = 0; i < XR; ++i) xreg[i] = src[i];
     };
@@ -1146,34 +1147,35 @@ double chunk_us(long long grid, int cps, int splits) {
     return us + (splits > 1 ? 4.5 : 0.0);
 }
 
+// dword_weights: every weight starts on a dword, which the tile kernel's copies to LDS
+// need (the chunk kernel loads weights from any address: 4096 x 4096 two bytes off, 512
+// tokens, Q4_0 69 us, Q8_0 82; the general kernel 100 and 129).
 // presplit: x's producer writes the split x (tile kernel only; no split launch).
-GemmPlan choose_plan(const LinearShape& s, bool x_aligned, bool presplit) {
+GemmPlan choose_plan(const LinearShape& s, bool dword_weights, bool presplit) {
     GemmPlan p;
     if (!chunk_supported(s) || static_cast<size_t>(s.M) * s.nb * block_bytes(s.qtype) >= (static_cast<size_t>(1) << 32)) return p;
     const size_t most = workspace_bytes(s);
     const int steps = s.nb / kTileBlocks;
     double best = 0.0;
-    if (x_aligned) {
-        ChunkCfg c = choose_chunk(s);
-        if (c.xs) {
-            c.xs = false;
-            c.tt = 2;
-            c.tok_tiles = (s.rows + 31) / 32;
-            c.npad = 32 * c.tok_tiles;
-            const long long tiles = static_cast<long long>(c.row_tiles) * c.tok_tiles;
-            c.splits = tiles >= 256 ? 1 : std::max(1, steps / 8);
-            c.cps = (steps + c.splits - 1) / c.splits;
-            c.splits = (steps + c.cps - 1) / c.cps;
-            if (c.splits > 1 && chunk_layout(s, c).total > most) c.splits = 1, c.cps = steps;
-        }
-        const long long grid = static_cast<long long>(c.row_tiles) * c.tok_tiles * c.splits;
-        if (chunk_layout(s, c).part_bytes < (static_cast<size_t>(1) << 31)) {
-            p.chunk = true;
-            p.c = c;
-            best = chunk_us(grid, c.cps, c.splits);
-            if (s.rows <= 16) return p;  // a quarter of a tile's tokens
-        }
+    ChunkCfg c = choose_chunk(s);
+    if (c.xs) {
+        c.xs = false;
+        c.tt = 2;
+        c.tok_tiles = (s.rows + 31) / 32;
+        c.npad = 32 * c.tok_tiles;
+        const long long tiles = static_cast<long long>(c.row_tiles) * c.tok_tiles;
+        c.splits = tiles >= 256 ? 1 : std::max(1, steps / 8);
+        c.cps = (steps + c.splits - 1) / c.splits;
+        c.splits = (steps + c.cps - 1) / c.cps;
+        if (c.splits > 1 && chunk_layout(s, c).total > most) c.splits = 1, c.cps = steps;
     }
+    if (chunk_layout(s, c).part_bytes < (static_cast<size_t>(1) << 31)) {
+        p.chunk = true;
+        p.c = c;
+        best = chunk_us(static_cast<long long>(c.row_tiles) * c.tok_tiles * c.splits, c.cps, c.splits);
+        if (s.rows <= 16) return p;  // a quarter of a tile's tokens
+    }
+    if (!dword_weights) return p;
     if (static_cast<size_t>(s.nb) * kTileN * 128 >= (static_cast<size_t>(1) << 31)) return p;
     p.row_tiles = (s.M + kTileM - 1) / kTileM;
     p.tok_tiles = (s.rows + kTileN - 1) / kTileN;
@@ -1197,8 +1199,6 @@ GemmPlan choose_plan(const LinearShape& s, bool x_aligned, bool presplit) {
     }
     return p;
 }
-
-bool x_on_16(const float* x) { return (reinterpret_cast<uintptr_t>(x) & 15u) == 0; }
 
 // Weights of a grouped call: n <= 3 linears with the same qtype, K and rows.
 struct ChunkGroup {
@@ -1317,10 +1317,9 @@ hipError_t launch_plan(const LinearShape& s, const GemmPlan& p, const float* x, 
     }
 }
 
-// The tile kernel's copies take weights that start on a dword.
-bool aligned_weights(const ChunkGroup& grp) {
+bool dword_aligned(int n, const void* const* w) {
     uintptr_t p = 0;
-    for (int g = 0; g < grp.n; ++g) p |= reinterpret_cast<uintptr_t>(grp.w[g]);
+    for (int g = 0; g < n; ++g) p |= reinterpret_cast<uintptr_t>(w[g]);
     return (p & 3u) == 0;
 }
 
@@ -1338,8 +1337,8 @@ hipError_t launch_gemm(const LinearShape& s, const void* w, const float* x, floa
     if (ws == nullptr) return hipErrorInvalidValue;
     char* base = static_cast<char*>(ws);
     const ChunkGroup grp{1, {w, nullptr, nullptr}, {y, nullptr, nullptr}, {s.M, 0, 0}};
-    const GemmPlan p = choose_plan(s, x_on_16(x), false);
-    if (p.chunk || (p.tile && aligned_weights(grp))) {
+    const GemmPlan p = choose_plan(s, dword_aligned(1, &w), false);
+    if (p.chunk || p.tile) {
         if (ws_bytes < workspace_bytes(s)) return hipErrorInvalidValue;
         return launch_plan(s, p, x, base, stream, grp, false);
     }
@@ -1353,17 +1352,16 @@ hipError_t launch_gemm(const LinearShape& s, const void* w, const float* x, floa
     }
 }
 
-GemmSplitX gemm_split_x(const LinearShape& s, int n, const int* M) {
+GemmSplitX gemm_split_x(const LinearShape& s, int n, const void* const* w, const int* M) {
     GemmSplitX r{};
-    if (n < 1 || n > 3 || M == nullptr) return r;
+    if (n < 1 || n > 3 || w == nullptr || M == nullptr) return r;
     LinearShape st = s;
     st.M = 0;
     for (int g = 0; g < n; ++g) {
         if (M[g] <= 0) return r;
         st.M += M[g];
     }
-    if (!chunk_supported(st)) return r;
-    const GemmPlan c = choose_plan(st, true, true);
+    const GemmPlan c = choose_plan(st, dword_aligned(n, w), true);
     if (!c.tile) return r;
     for (int g = 0; g + 1 < n; ++g)
         if (M[g] % kTileM != 0) return r;
@@ -1376,15 +1374,15 @@ GemmSplitX gemm_split_x(const LinearShape& s, int n, const int* M) {
     return r;
 }
 
-bool gemm_group_supported(const LinearShape& s, int n, const int* M, const float* x) {
-    if (n < 1 || n > 3 || M == nullptr) return false;
+bool gemm_group_supported(const LinearShape& s, int n, const void* const* w, const int* M) {
+    if (n < 1 || n > 3 || w == nullptr || M == nullptr) return false;
     LinearShape st = s;
     st.M = 0;
     for (int g = 0; g < n; ++g) {
         if (M[g] <= 0) return false;
         st.M += M[g];
     }
-    const GemmPlan p = choose_plan(st, x_on_16(x), false);
+    const GemmPlan p = choose_plan(st, dword_aligned(n, w), false);
     if (!p.tile && !p.chunk) return false;
     const int bm = p.tile ? kTileM : 64 * p.c.rw;
     for (int g = 0; g + 1 < n; ++g)
@@ -1401,22 +1399,21 @@ hipError_t launch_gemm_group(const LinearShape& s, int n, const void* const* w, 
         if (M[g] <= 0) return hipErrorInvalidValue;
         st.M += M[g];
     }
-    if (!x_split && !gemm_group_supported(s, n, M, x)) return hipErrorNotSupported;
-    const GemmPlan p = choose_plan(st, x_on_16(x), x_split);
+    if (!x_split && !gemm_group_supported(s, n, w, M)) return hipErrorNotSupported;
+    const GemmPlan p = choose_plan(st, dword_aligned(n, w), x_split);
     if (x_split && !p.tile) return hipErrorInvalidValue;  // gemm_split_x said no
     if (ws == nullptr) return hipErrorInvalidValue;
     if (ws_bytes < workspace_bytes(st)) return hipErrorInvalidValue;
     ChunkGroup grp{};
     grp.n = n;
     for (int g = 0; g < n; ++g) grp.w[g] = w[g], grp.y[g] = y[g], grp.M[g] = M[g];
-    if (p.tile && !aligned_weights(grp)) return hipErrorNotSupported;
     return launch_plan(st, p, x, static_cast<char*>(ws), stream, grp, x_split);
 }
 
-const char* gemm_kernel_name(const LinearShape& s) {
+const char* gemm_kernel_name(const LinearShape& s, bool dword_weights) {
     static thread_local char buf[96];
     const char* fmt = s.qtype == 1 ? "q8_0" : s.qtype == 2 ? "q4_0" : "q4_1";
-    const GemmPlan p = choose_plan(s, true, false);
+    const GemmPlan p = choose_plan(s, dword_weights, false);
     if (p.tile) {
         snprintf(buf, sizeof buf, "gemm_mfma_%s_tile_bm%d_bn%d_splitk%d", fmt, kTileM, kTileN, p.splits);
         return buf;

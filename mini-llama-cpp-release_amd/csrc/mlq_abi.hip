@@ -763,12 +763,12 @@ int mlq_hip_quant_linear_fused(const mlq_linear_call* calls, int n, void* stream
         // else one GEMM (or GEMV batch) per call.
         mlq::LinearShape total{w0->qtype, static_cast<int>(rows), w0->K, w0->nb, nrows};
         int M[3] = {0, 0, 0};
-        for (int i = 0; i < n && i < 3; ++i) M[i] = calls[i].w->M;
+        const void* wd[3] = {nullptr, nullptr, nullptr};
+        for (int i = 0; i < n && i < 3; ++i) M[i] = calls[i].w->M, wd[i] = calls[i].w->ptr;
         // The workspace is sized (and grown) only for a group that will launch.
-        if (n <= 3 && mlq::gemm_supported(total) && mlq::gemm_group_supported(total, n, M, calls[0].x)) {
-            const void* wd[3];
+        if (n <= 3 && mlq::gemm_supported(total) && mlq::gemm_group_supported(total, n, wd, M)) {
             float* yd[3];
-            for (int i = 0; i < n; ++i) wd[i] = calls[i].w->ptr, yd[i] = calls[i].y;
+            for (int i = 0; i < n; ++i) yd[i] = calls[i].y;
             const size_t need = mlq::gemm_workspace_bytes(total);
             void* ws = nullptr;
             if ((rc = stream_workspace(device, s, need, &ws)) != MLQ_OK) return rc;

@@ -114,14 +114,16 @@ bool gemm_supported(const LinearShape& s);
 size_t gemm_workspace_bytes(const LinearShape& s);
 hipError_t launch_gemm(const LinearShape& s, const void* w, const float* x, float* y, void* ws,
                        size_t ws_bytes, hipStream_t stream);
-const char* gemm_kernel_name(const LinearShape& s);
+// The kernel a call runs; dword_weights: the weights start on a dword.
+const char* gemm_kernel_name(const LinearShape& s, bool dword_weights = true);
 // Up to three linears that read the same x (same qtype, K and rows; e.g. q, k
 // and v of one layer) as one GEMM launch: linear g has M[g] rows and writes
 // y[g] ([rows][M[g]]); s.M is ignored (the total is the sum).  A row gets the
 // arithmetic of a single call of its linear, with the tile shape and K split
 // that the group's total M selects.
-// hipErrorNotSupported when the shape has no grouped path (no chunk kernel, or
-// a weight other than the last whose M is not a multiple of the tile height):
+// hipErrorNotSupported when the shape has no grouped path (neither the large-tile
+// nor the chunk kernel takes it, or a weight other than the last has an M that is
+// not a multiple of the tile height):
 // then launch the linears one by one.  The workspace is sized for a LinearShape
 // whose M is the total.
 // x_split: the workspace already holds x split as the GEMM reads it (written
@@ -131,9 +133,9 @@ hipError_t launch_gemm_group(const LinearShape& s, int n, const void* const* w, 
                              const float* x, void* ws, size_t ws_bytes, hipStream_t stream, bool x_split = false);
 // Whether launch_gemm_group would launch that group (rather than return
 // hipErrorNotSupported), so a caller sizes a workspace only when it will.
-bool gemm_group_supported(const LinearShape& s, int n, const int* M, const float* x);
+bool gemm_group_supported(const LinearShape& s, int n, const void* const* w, const int* M);
 
-// Where a grouped (or, n = 1, single) GEMM of `rows` > 128 token rows reads
+// Where a grouped (or, n = 1, single) GEMM that the large-tile kernel runs reads
 // its split x inside the workspace (xsplit_device.h's layout: xs [npad][nb][64]
 // halves, bsum [npad][nb], scale [npad]; byte offsets), and the workspace size
 // the launch needs.  ok = false: the call would not read a split x (the
@@ -143,7 +145,7 @@ struct GemmSplitX {
     int npad;
     size_t xs, bsum, scale, ws_bytes;
 };
-GemmSplitX gemm_split_x(const LinearShape& s, int n, const int* M);
+GemmSplitX gemm_split_x(const LinearShape& s, int n, const void* const* w, const int* M);
 
 // Persistent GEMV over a chain of linears (sequence.hip).  A stage is up to
 // kSeqMaxCalls GEMVs reading the same x; their rows are concatenated in call

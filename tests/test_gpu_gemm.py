@@ -86,7 +86,7 @@ def test_gemm_chunk_above_128_tokens(hip, orc, m, k, n):
 
 
 def test_gemm_large_tile_needs_dword_weights(hip, orc):
-    """Weights wrapped two bytes off a dword take the general kernel instead."""
+    """Weights wrapped two bytes off a dword take the chunk kernel instead."""
     m, k, n = 4097, 1664, 333
     rng = np.random.default_rng(31)
     x = rng.standard_normal((n, k), dtype=np.float32)
@@ -107,6 +107,42 @@ def test_gemm_large_tile_needs_dword_weights(hip, orc):
         check_close(y.download(np.float32, n * m).reshape(n, m), want, x, qt, blocks, f"qt={qt} unaligned weights")
         wt.free()
         buf.free()
+
+
+class Inside:
+    """A device buffer's bytes from an offset on, as the binding takes buffers."""
+
+    def __init__(self, hip, a, offset):
+        a = np.ascontiguousarray(a)
+        self.buf = hip.DeviceBuffer(a.nbytes + offset)
+        self.buf.upload(a, offset)
+        self.ptr, self.nbytes = self.buf.ptr + offset, a.nbytes
+
+
+@pytest.mark.parametrize("ms,k,n", [((4097,), 1664, 333), ((300,), 896, 40), ((300,), 896, 2), ((300,), 4160, 40),
+                                    ((256, 128, 72), 896, 40), ((4096, 4096, 300), 1664, 333)])
+def test_gemm_unaligned_operands(hip, orc, ms, k, n):
+    """Weights two bytes off a dword and x four off 16 bytes, each and both, one
+    linear or a group: the operands' addresses move no output past the bound."""
+    rng = np.random.default_rng(77)
+    x = rng.standard_normal((n, k), dtype=np.float32)
+    for fmt, qt in FMTS.items():
+        blocks = [orc.quantize(qt, rng.standard_normal((m, k), dtype=np.float32) * np.float32(0.02), threads=THREADS)
+                  for m in ms]
+        want = [orc.linear(qt, x, b, m, threads=THREADS) for b, m in zip(blocks, ms)]
+        for wo, xo in ((2, 0), (0, 4), (2, 4)):
+            print(f"gemm {fmt} Ms={ms} K={k} N={n} weights at +{wo} x at +{xo}", flush=True)
+            xb = Inside(hip, x, xo)
+            ws = [hip.Weight.wrap(qt, Inside(hip, b, wo), b.shape[0], m, k) for b, m in zip(blocks, ms)]
+            ys = [hip.DeviceBuffer(4 * n * m) for m in ms]
+            calls = hip.make_calls([(w, xb, y, n) for w, y in zip(ws, ys)])
+            if len(ms) > 1:
+                hip.linear_fused(calls)
+            else:
+                hip.linear_many(calls)
+            hip.synchronize(hip.stream(0))
+            for y, v, b, m in zip(ys, want, blocks, ms):
+                check_close(y.download(np.float32, n * m).reshape(n, m), v, x, qt, b, f"{fmt} M={m} +{wo} +{xo}")
 
 
 # The kernel of each shape: (out, in, rows, name part).
