@@ -71,7 +71,10 @@ __device__ __forceinline__ int slot_k(int g, int j) {
 // t, t + 256, ... (xsplit_device.h: two runs of four floats each).  The first
 // kXsCache of them stay in registers between the two passes (the max|x| of the
 // row, then the scaled split), so rows up to 16 384 elements are read once; longer
-// rows re-read the rest (L2 hits).  The split itself is xsplit_device.h's, which
+// rows re-read the rest (L2 hits).  A run is one float4 where every row starts on
+// 16 bytes (K a multiple of 4), four floats otherwise (whole calls of 64 weight rows,
+// floats / float4s, us: K = 4092, 2048 tokens 43.9 / 35.3; K = 32 704, 1024 tokens
+// 134 / 107).  The split itself is xsplit_device.h's, which
 // kernels producing a GEMM input also use.
 template <int QT, int C>
 __global__ __launch_bounds__(256) void xsplit_kernel(const float* __restrict__ x, int N, int K, int nb,
@@ -82,13 +85,18 @@ __global__ __launch_bounds__(256) void xsplit_kernel(const float* __restrict__ x
     const float* xr = x + static_cast<size_t>(valid ? n : 0) * K;
     __shared__ float red[4];
     const int items = 4 * nb;
-    const bool vec = K % 32 == 0 && (reinterpret_cast<uintptr_t>(xr) & 15u) == 0;  // K % 32: every row is like row 0
+    // Rows of whole runs on 16 bytes (K % 4: every row is like row 0); of whole blocks.
+    const bool quads = K % 4 == 0 && (reinterpret_cast<uintptr_t>(xr) & 15u) == 0;
+    const bool whole = quads && K % 32 == 0;
 
     auto load8 = [&](int i, float (&v)[8]) {
         const int k0 = xs_first<QT>(i), k1 = k0 + xs_second<QT>();
-        if (!valid || i >= items) {
 #pragma unroll
-            for (int k = 0; k < 8; ++k) v[k] = 0.0f;
+        for (int k = 0; k < 8; ++k) v[k] = 0.0f;
+        if (!valid || i >= items) return;
+        if (quads) {
+            if (k0 < K) xs_put4(v, 0, xr + k0);
+            if (k1 < K) xs_put4(v, 4, xr + k1);
         } else {
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
@@ -99,7 +107,7 @@ __global__ __launch_bounds__(256) void xsplit_kernel(const float* __restrict__ x
     };
 
     float cache[C][8];
-    if (vec) {
+    if (whole) {
         // Unconditional loads (items past the row re-read its last one): a load
         // under a branch is waited for at the join.
 #pragma unroll

@@ -145,6 +145,26 @@ def test_gemm_unaligned_operands(hip, orc, ms, k, n):
                 check_close(y.download(np.float32, n * m).reshape(n, m), v, x, qt, b, f"{fmt} M={m} +{wo} +{xo}")
 
 
+@pytest.mark.parametrize("k", [4092, 4090, 20032, 20476, 20474])
+@pytest.mark.parametrize("xo", [0, 4])
+def test_gemm_split_rows(hip, orc, k, xo):
+    """The x split of rows that are not whole blocks (whole float4s or not), and past
+    the 16 384 elements held in registers, from x on 16 bytes or on a float."""
+    m, n = 70, 33
+    rng = np.random.default_rng(k + xo)
+    x = rng.standard_normal((n, k), dtype=np.float32)
+    x[:, -3:] *= 50  # a row's maximum among its last elements
+    for fmt, qt in FMTS.items():
+        blocks = orc.quantize(qt, rng.standard_normal((m, k), dtype=np.float32) * np.float32(0.02), threads=THREADS)
+        print(f"gemm {fmt} M={m} K={k} N={n} x at +{xo}", flush=True)
+        wt, y = hip.Weight.upload(qt, blocks, m, k), hip.DeviceBuffer(4 * n * m)
+        wt.linear_device(Inside(hip, x, xo), y, rows=n)
+        hip.synchronize(hip.stream(0))
+        want = orc.linear(qt, x, blocks, m, threads=THREADS)
+        check_close(y.download(np.float32, n * m).reshape(n, m), want, x, qt, blocks, f"{fmt} K={k} +{xo}")
+        wt.free()
+
+
 # The kernel of each shape: (out, in, rows, name part).
 KERNELS = [(4097, 1664, 333, "_tile_"), (300, 896, 40, "_chunk_"), (300, 4160, 40, "_q4_1_bm")]
 
