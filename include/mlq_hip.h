@@ -371,7 +371,13 @@ int mlq_hip_rope(int device, float* x, int n_heads, int head_dim, int pos, float
  * q [n_heads][head_dim] over positions 0..pos of `layer` of a KV cache laid out
  * [n_layers][max_seq_len][n_kv_heads][head_dim] (CudaKVCache); scores scaled
  * by 1/sqrt(head_dim); query head h reads kv head h / (n_heads / n_kv_heads).
- * head_dim up to 512. */
+ * head_dim up to 512.  Long contexts (more than 49 152 elements of a head) are
+ * split over workgroups with scratch that the library lends to the stream: 16
+ * streams at a time per device.  The first 8 streams keep theirs until
+ * mlq_hip_stream_destroy; the other 8 pieces pass on once their last call is done.
+ * Calls on further streams with work in flight, on the per-thread default stream
+ * and under graph capture run one workgroup per head: same result up to the
+ * order of its f32 sums. */
 int mlq_hip_attention_decode(int device, const float* q, const float* keys, const float* values, int n_layers,
                              int layer, int max_seq_len, int n_heads, int n_kv_heads, int head_dim, int pos,
                              float* out, void* stream);

@@ -128,12 +128,25 @@ struct PickSlot {
 constexpr size_t kScratchBytes = size_t(48) << 20;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
-// Scratch of the decode attention op, one slot per stream that calls it outside
-// graph capture (the stream orders the slot's users; a recorded launch may be
-// replayed anywhere, so it gets none).  A fixed array: no allocation on any call.
-// Streams beyond the slots, and the per-thread default stream, whose one handle
-// stands for many streams, run the unsplit attention.
+// Scratch of the decode attention op for calls that split their positions: one
+// slot per stream, which orders the slot's users.  (A handle that the runtime gives
+// out again finds its slot free of work: hipStreamDestroy returns after the stream's
+// kernels, 100 ms for one of 100 ms.)  The first kAttnHeld streams keep their slots
+// until mlq_hip_stream_destroy; the other slots are lent:
+// their launches report completion in host memory (OpAttnScratch::done; 32 / 8 heads
+// of 128 at 3000 positions 13.7 -> 14.1 us a call), and one whose last launch is done
+// may go to another stream.  A fixed array: no allocation
+// on any call.  Recorded launches (replayed anywhere), the per-thread default stream
+// (one handle for many streams) and calls that find every slot in use run the
+// unsplit attention.
+struct AttnSlot {
+    hipStream_t stream = nullptr;
+    uint32_t seq = 0;             // lent slots: the last launch and its head groups
+    int groups = 0;
+    unsigned long long turn = 0;  // of its last use
+};
 constexpr int kAttnSlots = 16;
+constexpr int kAttnHeld = 8;
 static __device__ __align__(256) unsigned char attn_scratch[kAttnSlots][mlq::kOpAttnScratchBytes];
 
 struct DeviceState {
@@ -151,8 +164,11 @@ struct DeviceState {
     // x), so a retired buffer is kept until the process ends.
     std::vector<void*> retired_ws;
     std::vector<PickSlot> picks;
-    void* attn_scratch = nullptr;             // this device's address of `attn_scratch` (zeroed at set-up)
-    hipStream_t attn_slot[kAttnSlots] = {};  // the stream of each slot (guarded by ws_mu)
+    void* attn_scratch = nullptr;    // this device's address of `attn_scratch` (zeroed at set-up)
+    uint32_t* attn_done = nullptr;   // lent slots' completion words, pinned host memory
+    std::mutex attn_mu;              // guards the slots; held over a launch on a lent one
+    AttnSlot attn_slot[kAttnSlots];
+    unsigned long long attn_turn = 0;
     std::mutex pin_mu;         // guards the pinned stage of file uploads
     void* pin[2] = {nullptr, nullptr};
     hipEvent_t pin_done[2] = {nullptr, nullptr};
@@ -203,6 +219,13 @@ int ensure_device(int device) {
         if (st.init_err == hipSuccess) st.init_err = hipGetSymbolAddress(&st.attn_scratch, HIP_SYMBOL(attn_scratch));
         if (st.init_err == hipSuccess) {
             st.init_err = hipMemsetAsync(st.attn_scratch, 0, kAttnSlots * mlq::kOpAttnScratchBytes, st.stream);
+        }
+        if (st.init_err == hipSuccess) {
+            const size_t bytes = (kAttnSlots - kAttnHeld) * mlq::kOpAttnScratchGroups * sizeof(uint32_t);
+            void* words = nullptr;
+            st.init_err = hipHostMalloc(&words, bytes, hipHostMallocDefault);
+            if (st.init_err == hipSuccess) std::memset(words, 0, bytes);
+            st.attn_done = static_cast<uint32_t*>(words);
         }
         if (st.init_err == hipSuccess) st.init_err = hipStreamSynchronize(st.stream);
     });
@@ -365,19 +388,53 @@ int stream_pick(int device, hipStream_t stream, const char* caller, PickSlot* ou
     return MLQ_OK;
 }
 
-// The attention scratch of `stream`, or null (see attn_scratch).
-void* stream_attn_scratch(int device, hipStream_t stream) {
-    if (stream == hipStreamPerThread || capturing(stream)) return nullptr;
+// The slot for a launch on `stream`, or -1 (attn_mu is held).
+int attn_slot_for(DeviceState& st, hipStream_t stream) {
+    for (int i = 0; i < kAttnSlots; ++i)
+        if (st.attn_slot[i].stream == stream) return i;
+    for (int i = 0; i < kAttnHeld; ++i)
+        if (st.attn_slot[i].stream == nullptr) return i;
+    int best = -1;
+    for (int i = kAttnHeld; i < kAttnSlots; ++i) {
+        const AttnSlot& a = st.attn_slot[i];
+        const uint32_t* done = st.attn_done + (i - kAttnHeld) * mlq::kOpAttnScratchGroups;
+        bool idle = true;
+        for (int g = 0; g < a.groups && idle; ++g) idle = __atomic_load_n(done + g, __ATOMIC_ACQUIRE) == a.seq;
+        if (idle && (best < 0 || a.turn < st.attn_slot[best].turn)) best = i;
+    }
+    return best;
+}
+
+hipError_t attention_decode(int device, const float* q, const float* keys, const float* values, int layer, int max_seq_len,
+                            int n_heads, int n_kv_heads, int head_dim, int pos, float* out, hipStream_t s) {
+    const mlq::OpAttnPlan plan = mlq::op_attention_plan(q, keys, values, n_heads, n_kv_heads, head_dim, pos);
+    mlq::OpAttnScratch scratch;
+    auto launch = [&] {
+        return mlq::launch_op_attention_decode(q, keys, values, layer, max_seq_len, n_heads, n_kv_heads, head_dim, pos, out,
+                                               plan, scratch, s);
+    };
+    if (plan.splits == 1 || s == hipStreamPerThread || capturing(s)) return launch();
     DeviceState& st = g_dev[device];
-    std::lock_guard<std::mutex> lock(st.ws_mu);
-    int slot = -1;
-    for (int i = 0; i < kAttnSlots && slot < 0; ++i)
-        if (st.attn_slot[i] == stream) slot = i;
-    for (int i = 0; i < kAttnSlots && slot < 0; ++i)
-        if (st.attn_slot[i] == nullptr) slot = i;
-    if (slot < 0) return nullptr;
-    st.attn_slot[slot] = stream;
-    return static_cast<char*>(st.attn_scratch) + slot * mlq::kOpAttnScratchBytes;
+    std::unique_lock<std::mutex> lock(st.attn_mu);
+    const int i = attn_slot_for(st, s);
+    if (i < 0) {
+        lock.unlock();
+        return launch();
+    }
+    AttnSlot& a = st.attn_slot[i];
+    scratch.mem = static_cast<char*>(st.attn_scratch) + i * mlq::kOpAttnScratchBytes;
+    a.stream = s;
+    if (i < kAttnHeld) {
+        lock.unlock();
+        return launch();
+    }
+    // A lent slot: its launches are numbered in the order the stream runs them.  One
+    // that fails leaves the slot with its stream.
+    scratch.done = st.attn_done + (i - kAttnHeld) * mlq::kOpAttnScratchGroups;
+    scratch.seq = ++a.seq;
+    a.groups = plan.groups;
+    a.turn = ++st.attn_turn;
+    return launch();
 }
 
 int dispatch(int device, const mlq::LinearShape& s, const void* w, const float* x, float* y,
@@ -1020,9 +1077,9 @@ int mlq_hip_stream_destroy(void* stream) {
     if (stream == nullptr) return MLQ_OK;
     MLQ_HIP_CHECK(hipStreamSynchronize(static_cast<hipStream_t>(stream)));
     for (DeviceState& st : g_dev) {  // its attention slot, idle now, is free again
-        std::lock_guard<std::mutex> lock(st.ws_mu);
-        for (hipStream_t& s : st.attn_slot)
-            if (s == static_cast<hipStream_t>(stream)) s = nullptr;
+        std::lock_guard<std::mutex> lock(st.attn_mu);
+        for (AttnSlot& a : st.attn_slot)
+            if (a.stream == static_cast<hipStream_t>(stream)) a.stream = nullptr;
     }
     MLQ_HIP_CHECK(hipStreamDestroy(static_cast<hipStream_t>(stream)));
     return MLQ_OK;
@@ -1269,9 +1326,8 @@ int mlq_hip_attention_decode(int device, const float* q, const float* keys, cons
     if (rc == MLQ_OK) rc = check_device_ptr(values, device, caller, "value cache", cache);
     if (rc == MLQ_OK) rc = check_device_ptr(out, device, caller, "output", qb);
     if (rc != MLQ_OK) return rc;
-    const hipStream_t s = resolve_stream(device, stream);
-    hipError_t e = mlq::launch_op_attention_decode(q, keys, values, layer, max_seq_len, n_heads, n_kv_heads, head_dim,
-                                                   pos, out, stream_attn_scratch(device, s), s);
+    const hipError_t e = attention_decode(device, q, keys, values, layer, max_seq_len, n_heads, n_kv_heads, head_dim, pos,
+                                          out, resolve_stream(device, stream));
     return e == hipSuccess ? MLQ_OK : hip_fail(e, "op_attention_decode_kernel");
 }
 

@@ -227,11 +227,25 @@ constexpr int kOpSilu = 0;
 constexpr int kOpMul = 1;
 constexpr int kOpAdd = 2;
 constexpr int kOpAttnMaxHeadDim = 512;
-// Scratch that lets the attention split its positions over workgroups: arrival
-// counters (zero between launches), then the splits' states.  One launch at a time
-// may use it; null: one workgroup per head.
+// How a decode attention call runs: `groups` head groups of up to G heads, each
+// with its positions split over `splits` workgroups of `per` positions (1: one
+// workgroup per head).
+struct OpAttnPlan {
+    int G, groups, splits, per;
+};
+OpAttnPlan op_attention_plan(const float* q, const float* keys, const float* values, int n_heads, int n_kv_heads,
+                             int head_dim, int pos);
+// Scratch of a split launch: arrival counters (zero between launches), then the
+// splits' states.  One launch at a time may use it; mem null: the call runs
+// unsplit.  done (host memory, or null): the launch sets word g to seq as its last
+// use of head group g's part.
 constexpr int kOpAttnScratchGroups = 1024;
 constexpr size_t kOpAttnScratchBytes = size_t(1) << 20;
+struct OpAttnScratch {
+    void* mem = nullptr;
+    uint32_t* done = nullptr;
+    uint32_t seq = 0;
+};
 hipError_t launch_op_rmsnorm(const float* x, const float* w, int n, float eps, float* y, hipStream_t s);
 hipError_t launch_op_elementwise(int op, const float* a, const float* b, size_t n, float* y, hipStream_t s);
 hipError_t launch_op_softmax(const float* x, int n, float* y, hipStream_t s);
@@ -239,7 +253,8 @@ hipError_t launch_op_embedding(const float* table, int dim, int token, float* y,
 hipError_t launch_op_rope(float* x, int n_heads, int head_dim, int pos, float theta, bool neox, hipStream_t s);
 hipError_t launch_op_attention_decode(const float* q, const float* keys, const float* values, int layer,
                                       int max_seq, int n_heads, int n_kv_heads, int head_dim, int pos,
-                                      float* out, void* scratch, hipStream_t s);
+                                      float* out, const OpAttnPlan& plan, const OpAttnScratch& scratch,
+                                      hipStream_t s);
 hipError_t launch_op_matmul_f32(const float* a, const float* b, int m, int k, int n, bool b_transposed, float* c,
                                 hipStream_t s);
 

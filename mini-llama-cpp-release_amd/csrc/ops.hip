@@ -271,7 +271,8 @@ template <int LPR, int C, int G>
 __global__ __launch_bounds__(G == 1 ? 1024 : 256) void op_attention_split_kernel(const float* __restrict__ q, const float* __restrict__ keys,
                                           const float* __restrict__ values, int layer, int max_seq, int n_heads,
                                           int n_kv_heads, int hd, int pos, float scale2, float* __restrict__ out,
-                                          int per_split, float* __restrict__ part, unsigned* __restrict__ count) {
+                                          int per_split, float* __restrict__ part, unsigned* __restrict__ count,
+                                          uint32_t* done, uint32_t seq) {
     constexpr int R = 64 / LPR;    // rows of a wave
     constexpr int P = 2;           // rows of a lane in flight
     constexpr int E = 4 * C * LPR;  // head elements covered (>= hd)
@@ -444,8 +445,8 @@ __global__ __launch_bounds__(G == 1 ? 1024 : 256) void op_attention_split_kernel
     __shared__ unsigned last;
     __syncthreads();
     if (threadIdx.x == 0) {
-        const unsigned done = __hip_atomic_fetch_add(count + blockIdx.x, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        last = done == static_cast<unsigned>(splits) - 1 ? 1u : 0u;
+        const unsigned before = __hip_atomic_fetch_add(count + blockIdx.x, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        last = before == static_cast<unsigned>(splits) - 1 ? 1u : 0u;
     }
     __syncthreads();
     if (last == 0u) return;
@@ -513,6 +514,11 @@ __global__ __launch_bounds__(G == 1 ? 1024 : 256) void op_attention_split_kernel
         }
     }
     if (threadIdx.x == 0) __hip_atomic_store(count + blockIdx.x, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (done != nullptr) {
+        __syncthreads();                                  // every wave has used its part of the states
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the counter is back at zero
+        if (threadIdx.x == 0) __hip_atomic_store(done + blockIdx.x, seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
 }
 
 // C[M][N] = A[M][K] * op(B) in f32, op(B)[k][n] = B[k * N + n], or
@@ -603,12 +609,14 @@ hipError_t launch_op_rope(float* x, int n_heads, int head_dim, int pos, float th
 template <int G, int C>
 static void launch_attention_split(dim3 grid, int waves, const float* q, const float* keys, const float* values,
                                    int layer, int max_seq, int n_heads, int n_kv_heads, int hd, int pos, float scale,
-                                   float* out, int per_split, float* part, unsigned* count, hipStream_t s) {
+                                   float* out, int per_split, const OpAttnScratch& scratch, hipStream_t s) {
+    unsigned* const count = static_cast<unsigned*>(scratch.mem);
+    float* const part = scratch.mem != nullptr ? reinterpret_cast<float*>(count + kOpAttnScratchGroups) : nullptr;
     auto go = [&](auto kernel, int E) {
         const size_t lds = std::max(static_cast<size_t>(waves) * G * (E + 4) + G * (waves + 2),
                                     static_cast<size_t>(G) * 64 + 64 * waves * 4) * sizeof(float);
         hipLaunchKernelGGL(kernel, grid, dim3(64 * waves), lds, s, q, keys, values, layer, max_seq, n_heads, n_kv_heads,
-                           hd, pos, scale * 1.44269504f, out, per_split, part, count);
+                           hd, pos, scale * 1.44269504f, out, per_split, part, count, scratch.done, scratch.seq);
     };
     constexpr int F = 64 / (4 * C);  // lanes of a 64-element row
     if (hd <= 64) {
@@ -622,55 +630,67 @@ static void launch_attention_split(dim3 grid, int waves, const float* q, const f
     }
 }
 
+// 16-byte loads fit the head and the pointers.
+static bool attention_vectors(const float* q, const float* keys, const float* values, int head_dim) {
+    const uintptr_t p = reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(keys) | reinterpret_cast<uintptr_t>(values);
+    return head_dim % 4 == 0 && (p & 15u) == 0;
+}
+
+// Head elements that the lane layout of a head size covers.
+static int attention_elements(int head_dim) { return head_dim <= 64 ? 64 : head_dim <= 128 ? 128 : head_dim <= 256 ? 256 : 512; }
+
+// Positions split over workgroups where they outweigh the split's tail (about 5 us):
+// past 49 152 elements of a head (us, unsplit / split: 32 heads of 128 at 250 positions
+// 7.5 / 9.7, at 500 14.1 / 12.0; 14 heads of 64 at 1000 9.2 / 12.2, at 3000 34 / 14.7).
+// Workgroups of one head take 64 KB of cache, those of a group 128 KB, within 128 .. 768
+// (32 / 32 heads of 128, 3000 positions: 43.5 / 28.5 / 24.4 / 26.3 us with 256 / 512 /
+// 768 / 1024 workgroups; 32 / 8 heads: 14.9 / 15.8 / 18.4 with 128 / 256 / 512), and at
+// least 32 positions.
+OpAttnPlan op_attention_plan(const float* q, const float* keys, const float* values, int n_heads, int n_kv_heads,
+                             int head_dim, int pos) {
+    const int n = pos + 1;
+    OpAttnPlan p{1, n_heads, 1, n};
+    if (head_dim > kOpAttnMaxHeadDim || !attention_vectors(q, keys, values, head_dim)) return p;
+    if (static_cast<long long>(n) * head_dim <= 49152) return p;
+    const int group = n_heads / n_kv_heads;
+    const int G = group > 4 && head_dim <= 256 ? 8 : group >= 3 ? 4 : group;
+    const int groups = n_kv_heads * ((group + G - 1) / G);
+    if (groups > kOpAttnScratchGroups) return p;
+    const size_t bytes = static_cast<size_t>(n) * n_kv_heads * head_dim * 8;
+    const int target = static_cast<int>(std::min<size_t>(768, std::max<size_t>(128, bytes >> (G == 1 ? 16 : 17))));
+    const size_t room = kOpAttnScratchBytes - kOpAttnScratchGroups * sizeof(unsigned);
+    const size_t state = static_cast<size_t>(groups) * G * (attention_elements(head_dim) + 4) * sizeof(float);
+    const int splits = std::min({64, (target + groups - 1) / groups, n / 32, static_cast<int>(room / state)});
+    if (splits <= 1) return p;
+    const int per = (n + splits - 1) / splits;
+    return OpAttnPlan{G, groups, (n + per - 1) / per, per};
+}
+
 hipError_t launch_op_attention_decode(const float* q, const float* keys, const float* values, int layer,
                                       int max_seq, int n_heads, int n_kv_heads, int head_dim, int pos,
-                                      float* out, void* scratch, hipStream_t s) {
+                                      float* out, const OpAttnPlan& plan, const OpAttnScratch& scratch,
+                                      hipStream_t s) {
     const float scale = 1.0f / std::sqrt(static_cast<float>(head_dim));
     if (head_dim > kOpAttnMaxHeadDim) return hipErrorInvalidValue;
-    const uintptr_t p = reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(keys) | reinterpret_cast<uintptr_t>(values);
-    if (head_dim % 4 == 0 && (p & 15u) == 0) {
-        const int n = pos + 1;
-        const int group = n_heads / n_kv_heads;
-        // Positions split over workgroups where the caller lends scratch and they
-        // outweigh the split's tail (about 5 us): past 49 152 elements of a head (us,
-        // unsplit / split: 32 heads of 128 at 250 positions 7.5 / 9.7, at 500 14.1 /
-        // 12.0; 14 heads of 64 at 1000 9.2 / 12.2, at 3000 34 / 14.7).  Workgroups of one
-        // head take 64 KB of cache, those of a group 128 KB, within 128 .. 768 (32 / 32
-        // heads of 128, 3000 positions: 43.5 / 28.5 / 24.4 / 26.3 us with 256 / 512 / 768 /
-        // 1024 workgroups; 32 / 8 heads: 14.9 / 15.8 / 18.4 with 128 / 256 / 512), and at
-        // least 32 positions.
-        const int G = group > 4 && head_dim <= 256 ? 8 : group >= 3 ? 4 : group;
-        const int hgs = n_kv_heads * ((group + G - 1) / G);
-        const int E = head_dim <= 64 ? 64 : head_dim <= 128 ? 128 : head_dim <= 256 ? 256 : 512;
-        const size_t bytes = static_cast<size_t>(n) * n_kv_heads * head_dim * 8;
-        const int target = static_cast<int>(std::min<size_t>(768, std::max<size_t>(128, bytes >> (G == 1 ? 16 : 17))));
-        int splits = std::min({64, (target + hgs - 1) / hgs, n / 32});
-        if (static_cast<long long>(n) * head_dim <= 49152) splits = 1;
-        const size_t room = kOpAttnScratchBytes - kOpAttnScratchGroups * sizeof(unsigned);
-        splits = std::min<int>(splits, static_cast<int>(room / (static_cast<size_t>(hgs) * G * (E + 4) * sizeof(float))));
-        if (scratch != nullptr && splits > 1 && hgs <= kOpAttnScratchGroups) {
-            const int per = (n + splits - 1) / splits;
-            splits = (n + per - 1) / per;
-            unsigned* count = static_cast<unsigned*>(scratch);
-            float* part = reinterpret_cast<float*>(count + kOpAttnScratchGroups);
-            const dim3 grid(hgs, splits);
-            auto go = [&](auto launch) {
-                launch(grid, 4, q, keys, values, layer, max_seq, n_heads, n_kv_heads, head_dim, pos, scale, out, per, part,
-                       count, s);
-            };
-            switch (G) {
-                case 1: go(launch_attention_split<1, 4>); break;
-                case 2: go(launch_attention_split<2, 4>); break;
-                case 4: go(launch_attention_split<4, 4>); break;
-                default: go(launch_attention_split<8, 2>); break;
-            }
-            return hipGetLastError();
+    if (attention_vectors(q, keys, values, head_dim)) {
+        auto go = [&](auto launch, dim3 grid, int waves, int per, const OpAttnScratch& mem) {
+            launch(grid, waves, q, keys, values, layer, max_seq, n_heads, n_kv_heads, head_dim, pos, scale, out, per, mem, s);
+        };
+        const dim3 grid(plan.groups, plan.splits);
+        if (plan.splits == 1 || scratch.mem == nullptr) {
+            // One workgroup per head, as many waves as have rows.
+            const int rows = std::max(1, 64 / (attention_elements(head_dim) / 16));
+            const int waves = std::max(1, std::min(16, (pos + 2 * rows) / (2 * rows)));
+            go(launch_attention_split<1, 4>, dim3(n_heads, 1), waves, pos + 1, OpAttnScratch{});
+        } else if (plan.G == 1) {
+            go(launch_attention_split<1, 4>, grid, 4, plan.per, scratch);
+        } else if (plan.G == 2) {
+            go(launch_attention_split<2, 4>, grid, 4, plan.per, scratch);
+        } else if (plan.G == 4) {
+            go(launch_attention_split<4, 4>, grid, 4, plan.per, scratch);
+        } else {
+            go(launch_attention_split<8, 2>, grid, 4, plan.per, scratch);
         }
-        // One workgroup per head, as many waves as have rows.
-        const int rows = std::max(1, 64 / (E / 16));
-        const int waves = std::max(1, std::min(16, (n + 2 * rows - 1) / (2 * rows)));
-        launch_attention_split<1, 4>(dim3(n_heads, 1), waves, q, keys, values, layer, max_seq, n_heads, n_kv_heads, head_dim,
-                                     pos, scale, out, n, nullptr, nullptr, s);
         return hipGetLastError();
     }
     auto go = [&](auto kernel) {

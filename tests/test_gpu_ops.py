@@ -217,6 +217,113 @@ def test_attention_split(hip, stream):
                 hip.stream_destroy(sp)
 
 
+class Attention:
+    """One long-context attention: inputs, the reference, and calls with an output of
+    their own."""
+
+    def __init__(self, hip):
+        self.hip, self.shape, self.pos, self.seq = hip, (8, 4, 128), 1500, 1503
+        n_heads, n_kv, hd = self.shape
+        rng = np.random.default_rng(17)
+        K = rng.standard_normal((1, self.seq, n_kv, hd)).astype(np.float32)
+        V = rng.standard_normal((1, self.seq, n_kv, hd)).astype(np.float32)
+        q = rng.standard_normal((n_heads, hd)).astype(np.float32)
+        self.want = attention_ref(q, K, V, 0, self.pos, n_heads, n_kv, hd)
+        self.buf = [dev(hip, q), dev(hip, K), dev(hip, V)]
+
+    def call(self, stream, o):
+        n_heads, n_kv, hd = self.shape
+        q, k, v = self.buf
+        self.hip._check(self.hip.load().mlq_hip_attention_decode(0, q.ptr, k.ptr, v.ptr, 1, 0, self.seq, n_heads, n_kv, hd,
+                                                                 self.pos, o.ptr, stream))
+
+    def output(self):
+        return out(self.hip, self.want.size)
+
+    def result(self, o, what):
+        y = got(self.hip, o, self.want.size).reshape(self.want.shape)
+        close(y, self.want, what)
+        return y.tobytes()
+
+    def kinds(self):
+        """The bytes of a split and of an unsplit call (told apart by their rounding)."""
+        o = self.output()
+        self.call(None, o)
+        self.hip.synchronize()
+        split = self.result(o, "split")
+        sp = self.hip.stream_create(0)
+        g = self.hip.Graph.record(lambda: self.call(sp, o), sp)
+        g.launch(sp)
+        self.hip.synchronize(sp)
+        whole = self.result(o, "unsplit")
+        g.destroy()
+        self.hip.stream_destroy(sp)
+        assert split != whole
+        return split, whole
+
+
+class ForeignStreams:
+    """Streams of the HIP runtime, not of the library."""
+
+    def __init__(self, n):
+        self.rt = ctypes.CDLL("libamdhip64.so")
+        self.s = []
+        for _ in range(n):
+            p = ctypes.c_void_p()
+            assert self.rt.hipStreamCreateWithFlags(ctypes.byref(p), 1) == 0  # non-blocking, default priority
+            self.s.append(p.value)
+
+    def destroy(self):
+        for p in self.s:
+            assert self.rt.hipStreamSynchronize(ctypes.c_void_p(p)) == 0
+            assert self.rt.hipStreamDestroy(ctypes.c_void_p(p)) == 0
+        self.s = []
+
+
+def test_attention_scratch_passes_on(hip):
+    """Any number of streams get the split kernel, one after the other: streams the
+    library never sees destroyed, alive or gone, and its own."""
+    a = Attention(hip)
+    split, _ = a.kinds()
+    o = a.output()
+    say("attention scratch over many streams")
+    for round_ in range(2):
+        streams = ForeignStreams(24)
+        for i, s in enumerate(streams.s):
+            a.call(s, o)
+            hip.synchronize(s)
+            assert a.result(o, f"round {round_} foreign stream {i}") == split, (round_, i)
+            o.fill(0)
+        streams.destroy()
+    for i in range(24):
+        sp = hip.stream_create(0)
+        a.call(sp, o)
+        hip.synchronize(sp)
+        assert a.result(o, f"library stream {i}") == split, i
+        o.fill(0)
+        hip.stream_destroy(sp)
+
+
+def test_attention_streams_in_flight(hip):
+    """Calls in flight on more streams than there is scratch for, several on each, do
+    not meet in it: each result is a whole one, split or not."""
+    a = Attention(hip)
+    kinds = a.kinds()
+    streams = ForeignStreams(24)
+    say("attention on 24 streams in flight")
+    for round_ in range(3):
+        outs = [[a.output() for _ in range(3)] for _ in streams.s]
+        for j in range(3):
+            for s, o in zip(streams.s, outs):
+                a.call(s, o[j])
+        for s in streams.s:
+            hip.synchronize(s)
+        for i, o in enumerate(outs):
+            for j in range(3):
+                assert a.result(o[j], f"round {round_} stream {i} call {j}") in kinds
+    streams.destroy()
+
+
 def test_attention_split_infinities(hip):
     """A score of -inf (a masked key) drops out of a split softmax; a NaN key makes
     its heads NaN; an infinite v row past the position is not touched."""
