@@ -1044,41 +1044,36 @@ hipError_t launch_q(const LinearShape& s, const GemmCfg& c, const WsLayout& l, c
 //    reduction is a serial tail; short rows keep 2 chunks per split);
 //  * more: 128 rows x 32 tokens; 8 chunks per split unless the tiles alone give
 //    every CU a workgroup (then no K split).
-// Above 128 tokens the xs fields size the workspace only (workspace_bytes: the
-// shapes that fit a fixed scratch do not depend on which kernel runs).
 struct ChunkCfg {
     int rw, tt, row_tiles, tok_tiles, splits, cps, npad;
-    bool xs;
 };
 
 bool chunk_supported(const LinearShape& s) {
     return s.rows > 1 && s.nb >= 8 && s.nb % kChunkBlocks == 0 && s.K == s.nb * kQK && s.qtype >= 1 && s.qtype <= 3;
 }
 
+// Equal splits of `steps`, about `want` of them: how many, and the steps of each.
+void split_steps(int steps, int want, int* splits, int* each) {
+    *each = (steps + std::max(1, want) - 1) / std::max(1, want);
+    *splits = (steps + *each - 1) / *each;
+}
+
 ChunkCfg choose_chunk(const LinearShape& s) {
     ChunkCfg c;
-    c.rw = s.rows <= 16 ? 1 : 2;
-    c.tt = s.rows <= 16 ? 1 : (s.rows >= 512 && s.qtype == 1) ? 4 : 2;
-    c.xs = s.rows > 128;
+    c.rw = c.tt = s.rows <= 16 ? 1 : 2;
     c.row_tiles = (s.M + 64 * c.rw - 1) / (64 * c.rw);
     c.tok_tiles = (s.rows + 16 * c.tt - 1) / (16 * c.tt);
     c.npad = c.tok_tiles * 16 * c.tt;
     const long long tiles = static_cast<long long>(c.row_tiles) * c.tok_tiles;
     const int nchunks = s.nb / kChunkBlocks;
-    int splits;
+    int want = 1;
     if (c.tt == 1) {
-        splits = static_cast<int>((640 + tiles - 1) / tiles);
-        splits = std::min(splits, nchunks >= 16 ? nchunks / 4 : nchunks / 2);
-    } else if (!c.xs) {
-        splits = tiles >= 256 ? 1 : nchunks / 8;
-    } else {
-        const bool fill = c.tt == 4 ? tiles >= 256 : tiles >= 512;
-        splits = fill ? 1 : tiles >= 256 ? 2 : nchunks / 8;
+        if (tiles <= kGemmMaxTiles)
+            want = std::min(static_cast<int>((640 + tiles - 1) / tiles), nchunks >= 16 ? nchunks / 4 : nchunks / 2);
+    } else if (tiles < 256) {
+        want = nchunks / 8;
     }
-    splits = std::max(1, splits);
-    if (tiles > kGemmMaxTiles) splits = 1;
-    c.cps = (nchunks + splits - 1) / splits;
-    c.splits = (nchunks + c.cps - 1) / c.cps;
+    split_steps(nchunks, want, &c.splits, &c.cps);
     return c;
 }
 
@@ -1087,29 +1082,45 @@ struct ChunkWs {
     size_t xs, bsum, scale, part, part_bytes, total;
 };
 
-ChunkWs ws_layout(const LinearShape& s, bool xs, int npad, size_t part_bytes) {
+// npad: token rows of split x (0: the kernel splits x itself).
+ChunkWs ws_layout(const LinearShape& s, int npad, size_t part_bytes) {
     auto up = [](size_t v) { return (v + 255) & ~static_cast<size_t>(255); };
     ChunkWs l;
     l.xs = up(static_cast<size_t>(kGemmMaxTiles) * sizeof(unsigned));
-    l.bsum = l.xs + (xs ? up(static_cast<size_t>(s.nb) * npad * 64 * sizeof(_Float16)) : 0);
-    l.scale = l.bsum + (xs ? up(static_cast<size_t>(s.nb) * npad * sizeof(float)) : 0);
-    l.part = l.scale + (xs ? up(static_cast<size_t>(npad) * sizeof(float)) : 0);
+    l.bsum = l.xs + up(static_cast<size_t>(s.nb) * npad * 64 * sizeof(_Float16));
+    l.scale = l.bsum + up(static_cast<size_t>(s.nb) * npad * sizeof(float));
+    l.part = l.scale + up(static_cast<size_t>(npad) * sizeof(float));
     l.part_bytes = part_bytes;
     l.total = l.part + l.part_bytes;
     return l;
 }
 
 ChunkWs chunk_layout(const LinearShape& s, const ChunkCfg& c) {
-    return ws_layout(s, c.xs, c.npad,
+    return ws_layout(s, 0,
                      c.splits == 1 ? 0
                                    : static_cast<size_t>(c.row_tiles) * c.tok_tiles * c.splits *
                                          (c.rw * c.tt * kGemmThreads * 16));
 }
 
+// What a call's workspace holds at most; choose_plan keeps to it.  It is the general
+// kernel's need and, for the shapes that the other two take, the chunk kernel's own or,
+// above 128 tokens, a split x with the partials of 128-row tiles: of 64 tokens for
+// Q8_0 from 512 tokens and of 32 otherwise, with K in runs of 8 chunks below 256
+// tiles, in two above and whole once the chip is full.  A rule on the shape alone: it
+// says which calls fit the fixed scratch and a workspace that graphs were recorded
+// with, whichever kernel runs.
 size_t workspace_bytes(const LinearShape& s) {
-    size_t b = layout(s, choose(s)).total;
-    if (chunk_supported(s)) b = std::max(b, chunk_layout(s, choose_chunk(s)).total);
-    return b;
+    const size_t general = layout(s, choose(s)).total;
+    if (!chunk_supported(s)) return general;
+    if (s.rows <= 128) return std::max(general, chunk_layout(s, choose_chunk(s)).total);
+    const int bn = s.rows >= 512 && s.qtype == 1 ? 64 : 32;
+    const int tok_tiles = (s.rows + bn - 1) / bn;
+    const long long tiles = static_cast<long long>((s.M + 127) / 128) * tok_tiles;
+    const int steps = s.nb / kChunkBlocks;
+    int splits, each;
+    split_steps(steps, tiles >= (bn == 64 ? 256 : 512) ? 1 : tiles >= 256 ? 2 : steps / 8, &splits, &each);
+    const size_t part = splits == 1 ? 0 : static_cast<size_t>(tiles) * splits * (128 * bn * 4);
+    return std::max(general, ws_layout(s, bn * tok_tiles, part).total);
 }
 
 // Large-tile kernel: 128 rows x 64 tokens, eight waves as 2 row halves x 4
@@ -1166,17 +1177,7 @@ GemmPlan choose_plan(const LinearShape& s, bool dword_weights, bool presplit) {
     const int steps = s.nb / kTileBlocks;
     double best = 0.0;
     ChunkCfg c = choose_chunk(s);
-    if (c.xs) {
-        c.xs = false;
-        c.tt = 2;
-        c.tok_tiles = (s.rows + 31) / 32;
-        c.npad = 32 * c.tok_tiles;
-        const long long tiles = static_cast<long long>(c.row_tiles) * c.tok_tiles;
-        c.splits = tiles >= 256 ? 1 : std::max(1, steps / 8);
-        c.cps = (steps + c.splits - 1) / c.splits;
-        c.splits = (steps + c.cps - 1) / c.cps;
-        if (c.splits > 1 && chunk_layout(s, c).total > most) c.splits = 1, c.cps = steps;
-    }
+    if (c.splits > 1 && chunk_layout(s, c).total > most) c.splits = 1, c.cps = steps;
     if (chunk_layout(s, c).part_bytes < (static_cast<size_t>(1) << 31)) {
         p.chunk = true;
         p.c = c;
@@ -1190,11 +1191,11 @@ GemmPlan choose_plan(const LinearShape& s, bool dword_weights, bool presplit) {
     p.npad = p.tok_tiles * kTileN;
     const long long tiles = static_cast<long long>(p.row_tiles) * p.tok_tiles;
     for (int want = 1; want <= 16 && want <= steps; ++want) {
-        const int cps = (steps + want - 1) / want;
-        const int splits = (steps + cps - 1) / cps;
+        int splits, cps;
+        split_steps(steps, want, &splits, &cps);
         if (splits != want || (splits > 1 && (cps < 4 || tiles > kGemmMaxTiles))) continue;
         const size_t part = splits == 1 ? 0 : static_cast<size_t>(tiles) * splits * (kTileM * kTileN * 4);
-        const ChunkWs ws = ws_layout(s, true, p.npad, part);
+        const ChunkWs ws = ws_layout(s, p.npad, part);
         if (ws.total > most || part >= (static_cast<size_t>(1) << 31)) continue;
         const double us = tile_us(s, tiles * splits, cps, splits, !presplit, p.npad);
         if ((p.tile || p.chunk) && us >= best) continue;

@@ -29,7 +29,15 @@ def gemm():
     group.restype = ctypes.c_bool
     group.argtypes = [ctypes.POINTER(Shape), ctypes.c_int, ctypes.POINTER(ctypes.c_void_p), ctypes.POINTER(ctypes.c_int)]
 
+    need = lib._ZN3mlq20gemm_workspace_bytesERKNS_11LinearShapeE
+    need.restype = ctypes.c_size_t
+    need.argtypes = [ctypes.POINTER(Shape)]
+
     class Gemm:
+        @staticmethod
+        def workspace(qt, m, k, rows):
+            return need(ctypes.byref(Shape(qt, m, k, (k + 31) // 32, rows)))
+
         @staticmethod
         def kernel(qt, m, k, rows, dword=True):
             return name(ctypes.byref(Shape(qt, m, k, (k + 31) // 32, rows)), dword).decode()
@@ -75,3 +83,15 @@ def test_group_of_weights_off_a_dword(gemm, qt):
             name = gemm.kernel(qt, sum(ms), k, rows, at == 0)
             whole = nb % 4 == 0 and all(m % int(name.split("_bm")[1].split("_")[0]) == 0 for m in ms[:-1])
             assert gemm.grouped(qt, ms, k, rows, at) == whole, (rows, ms, k, at, name)
+
+
+@pytest.mark.parametrize("qt,m,k,rows,need", [
+    (oracle.Q4_0, 4096, 4096, 16, 2629888), (oracle.Q4_0, 4096, 4096, 128, 19202560),
+    (oracle.Q4_0, 4096, 4096, 129, 22381312), (oracle.Q8_0, 4096, 4096, 300, 26641664),
+    (oracle.Q8_0, 4096, 4096, 512, 25692160), (oracle.Q4_1, 11008, 4096, 512, 8914944),
+    (oracle.Q4_0, 12790, 384, 130, 16900352), (oracle.Q8_0, 2121, 11264, 292, 45769984),
+    (oracle.Q4_0, 300, 4160, 200, 7113728), (oracle.Q4_1, 70, 4092, 33, 1487104)])
+def test_workspace_of_a_shape_stays(gemm, qt, m, k, rows, need):
+    """A shape's workspace is part of the interface: it says which calls fit the fixed
+    scratch of mlq_hip_quant_linear_noalloc and a workspace that graphs recorded."""
+    assert gemm.workspace(qt, m, k, rows) == need
