@@ -625,7 +625,7 @@ static void launch_attention_split(dim3 grid, int waves, const float* q, const f
         go(op_attention_split_kernel<2 * F, C, G>, 128);
     } else if (hd <= 256) {
         go(op_attention_split_kernel<4 * F, C, G>, 256);
-    } else {
+    } else if constexpr (G < 8) {  // groups of 8 take heads of up to 256
         go(op_attention_split_kernel<8 * F, C, G>, 512);
     }
 }
