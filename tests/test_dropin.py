@@ -52,11 +52,20 @@ PROGRAMS = sorted({c[0] for c in CASES}) + ["mini-llama"]
 
 
 def _bin(name):
+    """The program, a skip where neither it nor the sources to build it are there, or,
+    with MLQ_EXPECT_DROPIN set, a failure instead."""
     path = os.path.join(OUT, name)
-    if not os.path.exists(path) and not os.path.isdir("/root/reference/src"):
+    buildable = os.path.isdir("/root/reference/src") or os.environ.get("MLQ_EXPECT_DROPIN")
+    if not os.path.exists(path) and not buildable:
         pytest.skip("reference programs not built (oracle/_ref) and their sources are absent")
     assert os.path.exists(path), "build it with `make -C oracle dropin` (needs the reference sources)"
     return path
+
+
+def test_missing_program_fails_where_expected(monkeypatch):
+    monkeypatch.setenv("MLQ_EXPECT_DROPIN", "1")
+    with pytest.raises(AssertionError, match="build it with"):
+        _bin("no-such-program")
 
 
 @pytest.mark.parametrize("name", PROGRAMS)
