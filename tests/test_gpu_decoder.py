@@ -321,3 +321,79 @@ def test_prefill_equals_steps(hip, orc, tmp_path, fmt):
     with pytest.raises(hip.MlqError, match="position out of range"):
         dec.forward(1, 1200)
     dec.close()
+
+
+def forward64(orc, hip, path, tokens, layers, heads, kv_heads, theta=10000.0, eps=1e-5):
+    """Logits at every position in 64 bits: a restatement of forward_batch for a llama
+    model (src/forward.cpp:496-700) from the file's own tensors."""
+    f = hip.GgufFile(path)
+    fmt = {8: oracle.Q8_0, 2: oracle.Q4_0, 3: oracle.Q4_1}
+    info = {t["name"]: t for t in f.tensors()}
+
+    def tensor(name):
+        t, raw = info[name], f.tensor_bytes(name)
+        if t["type"] == 0:
+            return raw.view(np.float32).astype(np.float64).reshape([int(d) for d in t["dims"]][::-1])
+        k, m = (int(d) for d in t["dims"])
+        qt = fmt[t["type"]]
+        blocks = raw.reshape(-1, oracle.BLOCK_BYTES[qt])
+        return orc.dequantize(qt, blocks, m, k).reshape(m, k).astype(np.float64)
+
+    def rms(x, w):
+        return x / np.sqrt((x * x).mean(-1, keepdims=True) + eps) * w
+
+    def rope(x):
+        hd = x.shape[-1]
+        a = np.arange(len(x))[:, None, None] * theta ** (-2 * np.arange(hd // 2) / hd)
+        even, odd = x[..., 0::2], x[..., 1::2]
+        return np.stack([even * np.cos(a) - odd * np.sin(a), even * np.sin(a) + odd * np.cos(a)], -1).reshape(x.shape)
+
+    x = tensor("token_embd.weight")[tokens]
+    n, hd = len(tokens), x.shape[1] // heads
+    hidden = np.arange(n)[None, :] > np.arange(n)[:, None]
+    for l in range(layers):
+        def w(name):
+            return tensor(f"blk.{l}.{name}.weight")
+
+        h = rms(x, w("attn_norm"))
+        q = rope((h @ w("attn_q").T).reshape(n, heads, hd))
+        k = rope((h @ w("attn_k").T).reshape(n, kv_heads, hd))
+        v = (h @ w("attn_v").T).reshape(n, kv_heads, hd)
+        att = np.empty_like(q)
+        for i in range(heads):
+            g = i // (heads // kv_heads)
+            s = np.where(hidden, -np.inf, q[:, i] @ k[:, g].T / np.sqrt(hd))
+            p = np.exp(s - s.max(-1, keepdims=True))
+            att[:, i] = p / p.sum(-1, keepdims=True) @ v[:, g]
+        x = x + att.reshape(n, -1) @ w("attn_output").T
+        h = rms(x, w("ffn_norm"))
+        g = h @ w("ffn_gate").T
+        x = x + (g / (1 + np.exp(-g)) * (h @ w("ffn_up").T)) @ w("ffn_down").T
+    return rms(x, tensor("output_norm.weight")) @ tensor("output.weight").T
+
+
+@pytest.mark.parametrize("fmt", ["q4_0", "q8_0", "q4_1"])
+def test_logits_in_64_bits(hip, orc, tmp_path, fmt):
+    """Prefill (large-tile GEMMs fed by the norm and SwiGLU kernels' split x) and steps
+    (split attention from 129 positions on) against a 64-bit forward of the same
+    file: the check that needs no reference build.  Bounds: f32 throughout is some 20
+    dependent operations, each the root of 88 blocks in roundings of 2^-24 (1e-5); the
+    one-row linears of Q4 weights (a step's, a prefill's last) take x as 16-bit integers
+    per block, 2^-16 of its largest (2e-5 a linear, 15 of them in a step)."""
+    bound = 2e-5 if fmt == "q8_0" else 3e-4
+    path = mf.write_model(orc, str(tmp_path / f"wide64_{fmt}.gguf"), layers=2, dim=2048, hidden=2816, heads=16, kv_heads=8,
+                          vocab=500, ctx=700, fmts=(fmt,), lm=fmt, seed=12, scale=0.02)
+    say(f"decoder {fmt} against 64 bits")
+    tokens = np.random.default_rng(4).integers(0, 500, 640)
+    want = forward64(orc, hip, path, tokens, 2, 16, 8)
+    dec = hip.Decoder(path)
+    for n in (2, 17, 64, 129, 300, 640):
+        worst = close(dec.prefill(tokens[:n]), want[n - 1], f"{fmt} prefill of {n}")
+        say(f"  prefill of {n}: {worst:.2e}")
+        assert worst <= bound
+    dec.prefill(tokens[:600])
+    for pos in range(600, 640):
+        worst = close(dec.forward(int(tokens[pos]), pos), want[pos], f"{fmt} step at {pos}")
+        assert worst <= bound
+    say(f"  step at 639: {worst:.2e}")
+    dec.close()

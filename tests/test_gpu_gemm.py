@@ -165,6 +165,81 @@ def test_gemm_split_rows(hip, orc, k, xo):
         wt.free()
 
 
+def close64(orc, got, x, qt, blocks, m, label):
+    """2-norm of the difference to the 64-bit product over the product's.  Every block
+    of a row adds one f32 rounding (2^-24, signs at random: the root of their number)
+    and the hi / lo halves carry 22 bits of x, so a lost lo half (2^-12) or a sum in
+    fewer bits shows where the 1e-3 of the other checks does not see it."""
+    k = x.shape[1]
+    want = x.astype(np.float64) @ orc.dequantize(qt, blocks, m, k).reshape(m, k).astype(np.float64).T
+    err = float(np.linalg.norm(got - want) / np.linalg.norm(want))
+    bound = np.sqrt(k / 32) * 2.0 ** -24 + 2.0 ** -22
+    print(f"{label}: {err:.2e} of {bound:.2e}", flush=True)
+    assert err <= bound, label
+
+
+@pytest.mark.parametrize("m,k,n,part", [(4097, 1664, 333, "_tile_"), (4097, 4096, 129, "_tile_"), (300, 896, 16, "_chunk_"),
+                                        (300, 896, 40, "_chunk_"), (300, 4160, 40, "_bm64_"), (300, 4160, 333, "_bm128_")])
+def test_gemm_against_64_bits(hip, orc, m, k, n, part):
+    """Each kernel's rounding, in every format."""
+    rng = np.random.default_rng(64)
+    x = rng.standard_normal((n, k), dtype=np.float32)
+    for fmt, qt in FMTS.items():
+        name = hip.kernel_name(qt, n, m, k)
+        assert part in name, name
+        blocks = orc.quantize(qt, rng.standard_normal((m, k), dtype=np.float32) * np.float32(0.02), threads=THREADS)
+        wt = hip.Weight.upload(qt, blocks, m, k)
+        close64(orc, wt.linear_host(x), x, qt, blocks, m, name)
+        wt.free()
+
+
+@pytest.mark.parametrize("ms,k,n", [((3072, 1000), 4096, 333),       # one split, a short last weight
+                                    ((2048, 256, 200), 4096, 333),   # two splits
+                                    ((1024, 1024, 72), 11008, 100)])  # seven
+def test_gemm_large_tile_group(hip, orc, ms, k, n):
+    """Two and three weights in one launch of the large-tile kernel: each row tile's
+    weight, output and size, with and without a K split."""
+    rng = np.random.default_rng(sum(ms))
+    x = rng.standard_normal((n, k), dtype=np.float32)
+    xb = hip.DeviceBuffer.from_array(x)
+    for fmt, qt in FMTS.items():
+        name = hip.kernel_name(qt, n, sum(ms), k)
+        assert "_tile_" in name and ("splitk1" in name) == (len(ms) == 2), name
+        blocks = [orc.quantize(qt, rng.standard_normal((m, k), dtype=np.float32) * np.float32(0.02), threads=THREADS)
+                  for m in ms]
+        ws = [hip.Weight.upload(qt, b, m, k) for b, m in zip(blocks, ms)]
+        ys = [hip.DeviceBuffer(4 * n * m) for m in ms]
+        print(f"gemm group {name} Ms={ms}", flush=True)
+        for _ in range(2):  # the second launch finds the counters that the first left
+            for y in ys:
+                y.fill(0xFF)
+            hip.linear_fused(hip.make_calls([(w, xb, y, n) for w, y in zip(ws, ys)]))
+            hip.synchronize()
+            for y, b, m in zip(ys, blocks, ms):
+                close64(orc, y.download(np.float32, n * m).reshape(n, m), x, qt, b, m, f"{fmt} M={m}")
+
+
+@pytest.mark.parametrize("m,k,n,part", [(4097, 1664, 333, "_tile_"), (300, 896, 40, "_chunk_")])
+def test_gemm_nonfinite_x(hip, orc, m, k, n, part):
+    """An infinity or a NaN in a token's x makes that token's outputs non-finite, as the
+    oracle's, and leaves every other token's bits alone."""
+    rng = np.random.default_rng(5)
+    x = rng.standard_normal((n, k), dtype=np.float32)
+    bad = x.copy()
+    bad[3, 5], bad[n - 1, k - 1], bad[n // 2, 64] = np.inf, np.nan, -np.inf
+    rows = [3, n // 2, n - 1]
+    for fmt, qt in FMTS.items():
+        assert part in hip.kernel_name(qt, n, m, k)
+        blocks = orc.quantize(qt, rng.standard_normal((m, k), dtype=np.float32) * np.float32(0.02), threads=THREADS)
+        print(f"gemm {fmt} M={m} K={k} N={n} with infinities", flush=True)
+        wt = hip.Weight.upload(qt, blocks, m, k)
+        clean, got = wt.linear_host(x), wt.linear_host(bad)
+        wt.free()
+        want = orc.linear(qt, bad[rows], blocks, m, threads=THREADS)
+        assert not np.isfinite(want).any() and not np.isfinite(got[rows]).any()
+        assert np.array_equal(np.delete(got, rows, axis=0), np.delete(clean, rows, axis=0))
+
+
 # The kernel of each shape: (out, in, rows, name part).
 KERNELS = [(4097, 1664, 333, "_tile_"), (300, 896, 40, "_chunk_"), (300, 4160, 40, "_q4_1_bm")]
 
