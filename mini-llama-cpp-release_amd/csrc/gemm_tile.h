@@ -3,12 +3,13 @@
 // fp16 hi + lo per token, weights as exact fp16 integers, one block of 32 k folded
 // into the f32 sums at a time with its scale).
 //
-// Bound: the matrix cores and the vector ALU about equally.  A block of a 32 x 32
-// tile costs 4 v_mfma_f32_32x32x16_f16 (128 cycles of a SIMD's matrix core; the
-// hi / lo split doubles the useful work) and 16 scale fmas, plus the decode of its
-// weights (10 VALU per 8 codes), which only a wide tile spreads out.  The same mix
-// of MFMA, fma and decode instructions without any memory access runs 4096 x 4096
-// at 512 tokens in 29 us (MFMA alone 22 us, at the 1.8-1.9 GHz the chip holds).
+// Bound: waits and issue order.  A block of a 32 x 32 tile costs 4
+// v_mfma_f32_32x32x16_f16 (128 cycles of a SIMD's matrix core; the hi / lo split
+// doubles the useful work) and 16 scale fmas, plus the decode of its weights (10 VALU
+// per 8 codes), which only a wide tile spreads out.  Counters at 4096 x 4096 Q4_0, 512
+// tokens: matrix cores 32 % busy, VALU 32 %, neither 50 %; LDS 26 %, 47 % of that in
+// bank conflicts; waves wait 30 % of their cycles and 34 % for issue.  The same mix of
+// MFMA, fma and decode instructions without any memory access takes 29 us.
 //
 // Split: a workgroup owns BM = 128 rows x BN = 64 tokens and eight waves (two per
 // SIMD).  Wave (wm, ks) computes a 64 x 64 tile of block ks of every step of four
@@ -28,9 +29,9 @@
 // sums stay f32 and an infinite m meets no padding.  64 cycles for two tiles, what
 // two fp16 instructions on the sums' halves took (call, us, halves / f32: 4096 x 4096
 // at 512 tokens 52.3 / 52.0, q/k/v at 2048 546 / 545, gate/up at 300 172.4 / 172.9).
-// Measured (kernel alone, us; the 128 x 32-token kernel it replaced in brackets):
-// 4096 x 4096, 512 tokens Q4_0 41.5 (58), Q8_0 48 (66), Q4_1 47 (75);
-// 11008 x 4096 Q4_0 128 (165).
+// Measured (kernel alone, cold weights, us; the 128 x 32-token kernel it replaced in
+// brackets): 4096 x 4096, 512 tokens Q4_0 43.0 (59.8), Q8_0 48.9 (68.6), Q4_1 51.0
+// (69.7); 11008 x 4096 Q4_0 122.6 (163.0).
 #pragma once
 
 #include "mlq_kernels.h"

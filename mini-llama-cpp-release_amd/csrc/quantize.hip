@@ -101,7 +101,7 @@ enum Rows { kWhole, kVector, kElement };
 // blocks of the workgroup (kQuantBlocks of them, a multiple of 16 bytes) gather in LDS
 // and leave in 16-byte stores.  One thread per block
 // (128-byte strides between lanes, 16-bit stores) / this, us: 11008 x 4096 Q8_0 46.3 /
-// 41.2 (5.5 TB/s; a copy runs at 5.1), Q4_0 39.2 / 38.2, Q4_1 40.4 / 40.4; 10000 x 2500 Q8_0
+// 41.2 (5.5 TB/s, four fifths of it reads; a copy, half writes, runs at 5.1), Q4_0 39.2 / 38.2, Q4_1 40.4 / 40.4; 10000 x 2500 Q8_0
 // 29.0 / 26.3; 16000 x 2051 Q4_0 69.7 / 58.7; 3000 x 896 Q4_0 5.2 / 4.1.
 template <int QT, Rows ROWS>
 __global__ __launch_bounds__(kQuantThreads) void quantize_kernel(const float* __restrict__ src,

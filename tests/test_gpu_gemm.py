@@ -46,7 +46,7 @@ def test_gemm_baseline_config4(hip, orc, shape, n):
 
 @pytest.mark.parametrize("shape", [(4096, 4096), (4096, 11008)], ids=lambda s: f"{s[0]}x{s[1]}")
 def test_gemm_256_tokens_two_splits(hip, orc, shape):
-    """256 token rows (x split once, 256 tiles: two K splits and their reduction)."""
+    """256 token rows: two K splits of the large-tile kernel and their reduction."""
     for fmt, qt in FMTS.items():
         name, _ = run(hip, orc, qt, *shape, 256)
         assert "splitk2" in name, name
@@ -55,7 +55,7 @@ def test_gemm_256_tokens_two_splits(hip, orc, shape):
 @pytest.mark.parametrize("m,k,n", [(4096, 4096, 16), (64, 64, 2), (33, 4096, 17), (300, 896, 40),
                                    (4864, 896, 7), (17, 64, 100), (1000, 11008, 3), (520, 4096, 130),
                                    (300, 896, 200), (200, 4096, 96),
-                                   # either side of the in-kernel x split (up to 128 token rows)
+                                   # either side of 128 token rows (the workspace rule changes there)
                                    (300, 4096, 128), (300, 4096, 129),
                                    # 130 blocks per row: not a whole number of 4-block chunks
                                    (300, 4160, 40), (300, 4160, 200)])
