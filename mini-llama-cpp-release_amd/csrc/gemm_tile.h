@@ -28,7 +28,8 @@
 // v_mfma_f32_32x32x1_2b_f32 (K = 1, both token tiles) per row tile and block: the
 // sums stay f32 and an infinite m meets no padding.  64 cycles for two tiles, what
 // two fp16 instructions on the sums' halves took (call, us, halves / f32: 4096 x 4096
-// at 512 tokens 52.3 / 52.0, q/k/v at 2048 546 / 545, gate/up at 300 172.4 / 172.9).
+// at 512 tokens 51.4 / 51.3, q/k/v at 2048 533 / 536, gate/up at 300 170.6 / 171.4;
+// at the other places of a step up to 2.7 % slower).
 // Measured (kernel alone, cold weights, us; the 128 x 32-token kernel it replaced in
 // brackets): 4096 x 4096, 512 tokens Q4_0 43.0 (59.8), Q8_0 48.9 (68.6), Q4_1 51.0
 // (69.7); 11008 x 4096 Q4_0 122.6 (163.0).
@@ -39,6 +40,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <type_traits>
 
 namespace mlq {
 namespace {
@@ -240,11 +242,16 @@ __global__ __launch_bounds__(64 * NWM * NWN * KS, (NWM * NWN * KS + 3) / 4) void
     uint32_t mask = 0x000F000Fu, mask4 = 0x00F000F0u, magic = 0x64006400u;
     asm volatile("" : "+v"(mask), "+v"(mask4), "+v"(magic));
 
-    // A row tile's sums: token tile t in elements 16 t .. 16 t + 15.
-    static_assert(WN == 2, "the block sums' product takes both token tiles");
-    f32x32 acc[WM];
+    // The sums of (row tile, token tile); Q4_1 keeps a row tile's two token tiles in one
+    // vector, as the block sums' product writes them.
+    static_assert(QT != 3 || WN == 2, "the block sums' product takes both token tiles");
+    using Acc = std::conditional_t<QT == 3, f32x32, f32x16>;
+    constexpr int AT = QT == 3 ? WN : 1;  // token tiles of one vector, 16 elements each
+    Acc acc[WM][WN / AT];
 #pragma unroll
-    for (int r = 0; r < WM; ++r) acc[r] = f32x32{};
+    for (int r = 0; r < WM; ++r)
+#pragma unroll
+        for (int t = 0; t < WN / AT; ++t) acc[r][t] = Acc{};
     const f32x16 zero{};
 
     // A step's operands of this wave: its blocks' decoded weights, scales and x.
@@ -334,14 +341,17 @@ __global__ __launch_bounds__(64 * NWM * NWN * KS, (NWM * NWN * KS + 3) / 4) void
             issue(c + ST, st_c, k, NT);
             if (r == WM - 1) read_x(st_n, j, t, nxt);
             const int kp = (k + NT - 1) % NT;  // the tile before
-            f32x32& ap = acc[kp % WM];
+            Acc& ap = acc[kp % WM][kp / WM / AT];
+            const int p0 = 16 * (kp / WM % AT);
 #pragma unroll
-            for (int i = 0; i < 16; ++i) ap[kp / WM * 16 + i] = __builtin_fmaf(dprev, C[(k + 1) & 1][i], ap[kp / WM * 16 + i]);
-            if (QT == 3 && k >= 1 && k <= WM) {
+            for (int i = 0; i < 16; ++i) ap[p0 + i] = __builtin_fmaf(dprev, C[(k + 1) & 1][i], ap[p0 + i]);
+            if constexpr (QT == 3) {
                 // + m * sum(x'), one k: both token tiles of a row tile (lanes 0-31 and
                 // 32-63 of the sums), between that row tile's two rounds of scale fmas.
-                const float m = static_cast<float>(__builtin_bit_cast(h2_t, cur.dm[kp % WM]).y);
-                ap = __builtin_amdgcn_mfma_f32_32x32x1f32(cur.s, m, ap, 0, 0, 0);
+                if (k >= 1 && k <= WM) {
+                    const float m = static_cast<float>(__builtin_bit_cast(h2_t, cur.dm[kp % WM]).y);
+                    ap = __builtin_amdgcn_mfma_f32_32x32x1f32(cur.s, m, ap, 0, 0, 0);
+                }
             }
             C[k & 1] = v;
             dprev = static_cast<float>(cur.d[r]);
@@ -374,9 +384,10 @@ __global__ __launch_bounds__(64 * NWM * NWN * KS, (NWM * NWN * KS + 3) / 4) void
             step(c, A, B);
             step(c + 1, B, A);
         }
-        f32x32& ap = acc[WM - 1];
+        Acc& ap = acc[WM - 1][(WN - 1) / AT];
+        constexpr int p0 = 16 * ((WN - 1) % AT);
 #pragma unroll
-        for (int i = 0; i < 16; ++i) ap[16 + i] = __builtin_fmaf(dprev, C[(WM * WN - 1) & 1][i], ap[16 + i]);
+        for (int i = 0; i < 16; ++i) ap[p0 + i] = __builtin_fmaf(dprev, C[(WM * WN - 1) & 1][i], ap[p0 + i]);
         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // no copy may land in the reduction below
     }
 
@@ -385,8 +396,9 @@ __global__ __launch_bounds__(64 * NWM * NWN * KS, (NWM * NWN * KS + 3) / 4) void
     constexpr int GR = T::G / T::RR, GKR = T::GK / T::RR;
     auto group_of = [&](int q) { return (q / GKR) * GR + ks * GKR + q % GKR; };
     auto acc4 = [&](int g) {
-        const f32x32& v = acc[g / 4 / WN];
-        const int i = 16 * (g / 4 % WN) + 4 * (g % 4);
+        const int t = g / 4 % WN;
+        const Acc& v = acc[g / 4 / WN][t / AT];
+        const int i = 16 * (t % AT) + 4 * (g % 4);
         return f32x4{v[i], v[i + 1], v[i + 2], v[i + 3]};
     };
     f32x4 own[T::GK];
